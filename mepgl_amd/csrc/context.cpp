@@ -16,6 +16,7 @@
 
 #include "../../include/mepgl.h"
 #include "common.hpp"
+#include "field_io.hpp"
 #include "gauge_local.hpp"
 #include "kernels.hpp"
 
@@ -117,6 +118,7 @@ struct mepgl_ctx {
   // host after an event that follows the writing launch.
   int* health = nullptr;
   hipEvent_t iter_done[2] = {nullptr, nullptr};
+  FieldIo io;                // workspace of the host transfers
 
   bool fp32() const { return precision == MEPGL_MIXED; }
 };
@@ -698,82 +700,49 @@ int reset_solver(mepgl_ctx* c) {
 
 bool valid_string(mepgl_ctx* c, int s) { return c && s >= 0 && s < (int)c->strings.size(); }
 
-// Field conversion between the host layout (F, N, N, 2) and the device planes.
-template <class T>
-void pack_fields(const StringHost& s, const double* a, const double* p1, const double* p2,
-                 std::vector<T>& out) {
-  const DevString& d = s.dev;
-  const int N = d.N, P = d.pitch, F = d.F;
-  out.assign((size_t)F * d.image_stride, (T)0);
-  const double* src[3] = {a, p1, p2};
-  for (int n = 0; n < F; ++n)
-    for (int f = 0; f < 1 + d.nc; ++f) {
-      if (!src[f]) continue;
-      for (int comp = 0; comp < 2; ++comp) {
-        T* dst = out.data() + (size_t)n * d.image_stride + (size_t)(2 * f + comp) * d.plane_stride;
-        const double* sp = src[f] + (size_t)n * N * N * 2;
-        for (int j = 0; j < N; ++j)
-          for (int i = 0; i < N; ++i) dst[(size_t)j * P + i] = (T)sp[((size_t)j * N + i) * 2 + comp];
-      }
-    }
+// The streams a transfer of host fields may use, once they are idle.
+struct IoStreams {
+  hipStream_t s[kMaxParts];
+};
+
+int io_streams(mepgl_ctx* c, IoStreams* io) {
+  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  for (int p = 0; p < kMaxParts; ++p) io->s[p] = part_stream(c, p);
+  return MEPGL_OK;
 }
 
-template <class T>
-void unpack_fields(const StringHost& s, const std::vector<T>& in, double* a, double* p1,
-                   double* p2) {
-  const DevString& d = s.dev;
-  const int N = d.N, P = d.pitch, F = d.F;
-  double* dst[3] = {a, p1, p2};
-  for (int n = 0; n < F; ++n)
-    for (int f = 0; f < 3; ++f) {
-      if (!dst[f]) continue;
-      for (int comp = 0; comp < 2; ++comp) {
-        double* dp = dst[f] + (size_t)n * N * N * 2;
-        if (f > d.nc) {
-          for (int j = 0; j < N; ++j)
-            for (int i = 0; i < N; ++i) dp[((size_t)j * N + i) * 2 + comp] = 0.0;
-          continue;
-        }
-        const T* sp = in.data() + (size_t)n * d.image_stride + (size_t)(2 * f + comp) * d.plane_stride;
-        for (int j = 0; j < N; ++j)
-          for (int i = 0; i < N; ++i) dp[((size_t)j * N + i) * 2 + comp] = (double)sp[(size_t)j * P + i];
-      }
-    }
+// The host arrays A, psi_1 and psi_2 of a string (psi_2 only with two
+// components).
+int host_fields(const StringHost& s, const double* a, const double* p1, const double* p2,
+                HostField (&f)[3]) {
+  int n = 0;
+  f[n++] = {const_cast<double*>(a), PAX, 2};
+  f[n++] = {const_cast<double*>(p1), PU1, 2};
+  if (s.dev.nc == 2 && p2) f[n++] = {const_cast<double*>(p2), PU2, 2};
+  return n;
 }
 
 int copy_out_fields(mepgl_ctx* c, int si, const void* dev, double* a, double* p1, double* p2) {
   StringHost& s = c->strings[si];
-  const size_t n = (size_t)s.dev.F * s.dev.image_stride;
-  if (c->fp32()) {
-    std::vector<float> h(n);
-    HIP_TRY(c, hipMemcpyAsync(h.data(), dev, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    unpack_fields(s, h, a, p1, p2);
-  } else {
-    std::vector<double> h(n);
-    HIP_TRY(c, hipMemcpyAsync(h.data(), dev, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    unpack_fields(s, h, a, p1, p2);
-  }
+  IoStreams io;
+  if (int rc = io_streams(c, &io)) return rc;
+  HostField f[3];
+  const int nf = host_fields(s, a, p1, p2, f);
+  HIP_TRY(c, download_fields(c->io, s.dev, dev, c->fp32(), f, nf, io.s, kMaxParts, c->device));
+  if (p2 && s.dev.nc == 1)
+    std::memset(p2, 0, sizeof(double) * 2 * (size_t)s.dev.F * s.dev.N * s.dev.N);
   return MEPGL_OK;
 }
 
-// Host fields (F, N, N, 2) into a device field set of one string.
-int copy_in_fields(mepgl_ctx* c, int si, void* dev, const double* a, const double* p1,
-                   const double* p2) {
+// Host fields (F, N, N, 2) into one or two device field sets of a string.
+int copy_in_fields(mepgl_ctx* c, int si, void* const* dev, int ndev, const double* a,
+                   const double* p1, const double* p2) {
   StringHost& s = c->strings[si];
-  const size_t n = (size_t)s.dev.F * s.dev.image_stride;
-  if (c->fp32()) {
-    std::vector<float> h;
-    pack_fields(s, a, p1, s.dev.nc == 2 ? p2 : nullptr, h);
-    HIP_TRY(c, hipMemcpyAsync(dev, h.data(), n * sizeof(float), hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-  } else {
-    std::vector<double> h;
-    pack_fields(s, a, p1, s.dev.nc == 2 ? p2 : nullptr, h);
-    HIP_TRY(c, hipMemcpyAsync(dev, h.data(), n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-  }
+  IoStreams io;
+  if (int rc = io_streams(c, &io)) return rc;
+  HostField f[3];
+  const int nf = host_fields(s, a, p1, p2, f);
+  HIP_TRY(c, upload_fields(c->io, s.dev, dev, ndev, c->fp32(), f, nf, io.s, kMaxParts, c->device));
   return MEPGL_OK;
 }
 
@@ -1293,6 +1262,7 @@ void mepgl_destroy(mepgl_ctx* c) {
   for (auto e : c->timing.pool) (void)hipEventDestroy(e);
   for (auto e : c->iter_done)
     if (e) (void)hipEventDestroy(e);
+  c->io.release();
   if (c->health) (void)hipHostFree(c->health);
   for (int* p : c->d_part_imgs)
     if (p) (void)hipFree(p);
@@ -1317,33 +1287,14 @@ int mepgl_upload(mepgl_ctx* c, int si, const double* a, const double* p1, const 
   // A NO_SELF_FIELD string whose A is the same in every image keeps one A
   // for all of them (image 0's planes); any other keeps A per image.
   if (s.dev.nsf) {
-    const size_t img = (size_t)s.dev.N * s.dev.N * 2;
-    bool same = true;
-    for (int k = 1; k < s.dev.F && same; ++k)
-      same = std::memcmp(a, a + (size_t)k * img, img * sizeof(double)) == 0;
+    const bool same = images_equal(a, s.dev.F, (size_t)s.dev.N * s.dev.N * 2);
     if ((int)same != s.dev.a_shared) {
       s.dev.a_shared = same ? 1 : 0;
       destroy_graphs(c);
       if ((rc = upload_descriptors(c))) return rc;
     }
   }
-  const size_t n = (size_t)s.dev.F * s.dev.image_stride;
-  for (int b = 0; b < 2; ++b) {
-    if (c->fp32()) {
-      std::vector<float> h;
-      pack_fields(s, a, p1, s.dev.nc == 2 ? p2 : nullptr, h);
-      HIP_TRY(c, hipMemcpyAsync(s.dev.x[b], h.data(), n * sizeof(float), hipMemcpyHostToDevice,
-                                c->stream));
-      HIP_TRY(c, hipStreamSynchronize(c->stream));
-    } else {
-      std::vector<double> h;
-      pack_fields(s, a, p1, s.dev.nc == 2 ? p2 : nullptr, h);
-      HIP_TRY(c, hipMemcpyAsync(s.dev.x[b], h.data(), n * sizeof(double), hipMemcpyHostToDevice,
-                                c->stream));
-      HIP_TRY(c, hipStreamSynchronize(c->stream));
-    }
-  }
-  return MEPGL_OK;
+  return copy_in_fields(c, si, s.dev.x, 2, a, p1, p2);
 }
 
 int mepgl_download(mepgl_ctx* c, int si, double* a, double* p1, double* p2) {
@@ -1447,25 +1398,13 @@ int mepgl_compute_jb(mepgl_ctx* c, int si, double* b, double* j1, double* j2) {
   if ((rc = run_aux(c, a, kKernelJB, 0))) return rc;
   StringHost& s = c->strings[si];
   const DevString& d = s.dev;
-  std::vector<double> h((size_t)d.F * d.image_stride);
-  HIP_TRY(c, hipMemcpyAsync(h.data(), s.jb, h.size() * sizeof(double), hipMemcpyDeviceToHost,
-                            c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  const int N = d.N, P = d.pitch;
-  for (int n = 0; n < d.F; ++n) {
-    const double* base = h.data() + (size_t)n * d.image_stride;
-    for (int j = 0; j < N; ++j)
-      for (int i = 0; i < N; ++i) {
-        const size_t o = (size_t)j * P + i, q = (size_t)n * N * N + (size_t)j * N + i;
-        b[q] = base[o];
-        j1[2 * q] = base[d.plane_stride + o];
-        j1[2 * q + 1] = base[2 * d.plane_stride + o];
-        if (j2) {
-          j2[2 * q] = d.nc == 2 ? base[3 * d.plane_stride + o] : 0.0;
-          j2[2 * q + 1] = d.nc == 2 ? base[4 * d.plane_stride + o] : 0.0;
-        }
-      }
-  }
+  // b and j are stored in double in both precisions.
+  IoStreams io;
+  if ((rc = io_streams(c, &io))) return rc;
+  const bool two = d.nc == 2 && j2;
+  const HostField f[3] = {{b, 0, 1}, {j1, 1, 2}, {j2, 3, 2}};
+  HIP_TRY(c, download_fields(c->io, d, s.jb, false, f, two ? 3 : 2, io.s, kMaxParts, c->device));
+  if (j2 && d.nc == 1) std::memset(j2, 0, sizeof(double) * 2 * (size_t)d.F * d.N * d.N);
   return MEPGL_OK;
 }
 
@@ -1770,7 +1709,7 @@ int mepgl_upload_state(mepgl_ctx* c, int si, int which, const double* a, const d
   if (rc) return rc;
   const DevString& d = c->strings[si].dev;
   void* dst = which == 0 ? d.g[0] : which == 1 ? d.g[1] : d.d[c->dp];
-  return copy_in_fields(c, si, dst, a, p1, p2);
+  return copy_in_fields(c, si, &dst, 1, a, p1, p2);
 }
 
 int mepgl_set_scalars(mepgl_ctx* c, int si, int which, const double* in) {

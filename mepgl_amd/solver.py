@@ -125,17 +125,27 @@ class Solver:
         N = self.strings[i].N
         return (self.F[i], N, N, 2)
 
+    def _field_arrays(self, i):
+        """Arrays for A, psi_1 and psi_2 of string i, and psi_2 for the library
+        to write: with one component psi_2 is zero, and its pages are never
+        touched."""
+        a, p1 = np.empty(self._shape(i)), np.empty(self._shape(i))
+        if self.strings[i].multicomponent:
+            p2 = np.empty(self._shape(i))
+            return a, p1, p2, p2
+        return a, p1, np.zeros(self._shape(i)), None
+
     def download(self, i: int):
         """Current fields (a, psi_1, psi_2) of string i, float64 (F, N, N, 2)."""
-        a, p1, p2 = (np.empty(self._shape(i)) for _ in range(3))
-        self._check(self._L.mepgl_download(self._ctx, i, _ptr(a), _ptr(p1), _ptr(p2)))
+        a, p1, p2, w2 = self._field_arrays(i)
+        self._check(self._L.mepgl_download(self._ctx, i, _ptr(a), _ptr(p1), _ptr(w2)))
         return a, p1, p2
 
     def download_state(self, i: int, which: str):
         """Solver buffers: "g" (caller's g), "g_old", "d" (direction)."""
         k = {"g": 0, "g_old": 1, "d": 2}[which]
-        a, p1, p2 = (np.empty(self._shape(i)) for _ in range(3))
-        self._check(self._L.mepgl_download_state(self._ctx, i, k, _ptr(a), _ptr(p1), _ptr(p2)))
+        a, p1, p2, w2 = self._field_arrays(i)
+        self._check(self._L.mepgl_download_state(self._ctx, i, k, _ptr(a), _ptr(p1), _ptr(w2)))
         return a, p1, p2
 
     def upload_state(self, i: int, which: str, a, p1, p2=None):
@@ -220,16 +230,19 @@ class Solver:
 
     def gradient(self, i: int):
         """gradientPsi + gradientA (nlcg.cu:504-888) at the current fields."""
-        a, p1, p2 = (np.empty(self._shape(i)) for _ in range(3))
-        self._check(self._L.mepgl_gradient(self._ctx, i, _ptr(a), _ptr(p1), _ptr(p2)))
+        a, p1, p2, w2 = self._field_arrays(i)
+        self._check(self._L.mepgl_gradient(self._ctx, i, _ptr(a), _ptr(p1), _ptr(w2)))
         return a, p1, p2
 
     def computeJB(self, i: int):
         """computeJB (nlcg.cu:367-380): b (F, N, N), j_1 and j_2 (F, N, N, 2)."""
         N = self.strings[i].N
         b = np.empty((self.F[i], N, N))
-        j1, j2 = np.empty(self._shape(i)), np.empty(self._shape(i))
-        self._check(self._L.mepgl_compute_jb(self._ctx, i, _ptr(b), _ptr(j1), _ptr(j2)))
+        j1 = np.empty(self._shape(i))
+        two = self.strings[i].multicomponent
+        j2 = np.empty(self._shape(i)) if two else np.zeros(self._shape(i))
+        self._check(self._L.mepgl_compute_jb(self._ctx, i, _ptr(b), _ptr(j1),
+                                             _ptr(j2) if two else None))
         return b, j1, j2
 
     def nlcgSteps(self, iter_n: int, nlcg: bool = True, maxwell_solver: bool = False):
