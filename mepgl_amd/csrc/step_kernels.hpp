@@ -719,13 +719,21 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
   constexpr bool nsf = NSF;
   const bool exact = s.poly_exact;
   const bool store = t.i < N;
-  const T idx = (T)s.inv_dx, dx2 = (T)s.dx2;
+  const T dx = (T)s.dx, dx2 = (T)s.dx2;
   const T eta = (T)s.eta, gam = (T)s.gamma, del = (T)s.delta;
-  CompConst<T> kconst[NC];
-  if (!PL) load_comp_const<T, NC>(s, 0, kconst);
+  // The constants of uniform parameters stay in scalar registers.
+  PolyConst<T, NC> pconst;
+  if constexpr (!PL) {
+    CompConst<T> kconst[NC];
+    load_comp_const<T, NC>(s, 0, kconst);
+    pconst = poly_const<T, NC>(kconst, eta, gam, del, dx, dx2, exact);
+    T* const v = (T*)&pconst;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(pconst) / sizeof(T)); ++i) v[i] = uniform_value(v[i]);
+  }
   const ParamView<NC> pv = param_view<NC>(s);
   gptr<const double> __restrict__ hp = as_global(s.h.p);
-  const T hv = (T)s.h.v;
+  const T hv = (T)s.h.v * dx;
   double acc_s[5] = {0, 0, 0, 0, 0}, acc_c[5] = {0, 0, 0, 0, 0};
   // Everything the march needs from the string's descriptor is read above,
   // before the branch and before any store, so it stays in scalar registers.
@@ -817,19 +825,18 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
         nb.du[q][2] = wpl.du[q];
         nb.dv[q][2] = wpl.dv[q];
       }
-      CompConst<T> k[NC];
+      PolyConst<T, NC> pc = pconst;
+      nb.h0 = hv;
       if constexpr (PL) {
+        CompConst<T> k[NC];
         comp_from_params<T, NC>(rp[IC].prm, pv.q, k);
-        nb.h0 = hp ? rp[IC].h[0] : hv;
-      } else {
-#pragma unroll
-        for (int q = 0; q < NC; ++q) k[q] = kconst[q];
-        nb.h0 = hv;
+        pc = poly_const<T, NC>(k, eta, gam, del, dx, dx2, exact);
+        if (hp) nb.h0 = rp[IC].h[0] * dx;
       }
 
       if (live) {
         const Quartic<T> qv =
-            site_poly<T, NC>(nb, k, eta, gam, del, idx, dx2, wc.nn & 0xff, wc.nn >> 8, nsf, exact);
+            site_poly<T, NC>(nb, pc, wc.nn & 0xff, wc.nn >> 8, nsf);
 #pragma unroll
         for (int r = 0; r < 5; ++r) acc_s[r] += (double)qv.c[r];
       }
