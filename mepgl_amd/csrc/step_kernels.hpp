@@ -10,8 +10,8 @@
 // even segments, up in odd ones), keeping the rows j-1, j, j+1 it needs in a
 // register window and prefetching the next-but-one row while it computes
 // row j.  Neighbours along x come from the adjacent lanes through DPP wave
-// shifts; the two columns just outside the strip are loaded by lanes 0 and
-// 63 only.  Every field value is therefore read from HBM once per launch,
+// shifts; the two columns just outside the strip come through a ring in LDS
+// (HaloPlan).  Every field value is therefore read from HBM once per launch,
 // plus the halo rows and columns the strip shares with its neighbours,
 // which L2 serves: adjacent work items run at the same time on the same
 // XCD, and neighbouring segments reach their shared rows together.
@@ -106,67 +106,121 @@ constexpr int step_waves() {
 template <int W>
 __device__ __forceinline__ int step_item(int nitems) {
   const int groups = (nitems + W - 1) / W;
-  return xcd_item(blockIdx.x, groups) * W + (W > 1 ? (int)(threadIdx.x / kWave) : 0);
+  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave)) : 0;
+  return xcd_item(blockIdx.x, groups) * W + wave;
 }
 
-// Edge columns traded inside a workgroup.  The W items of a workgroup are
-// consecutive in the work list: horizontally adjacent strips of one segment
-// (or of two, when a row has fewer than W strips).  A strip's halo columns
-// are then its neighbours' edge columns, which the neighbours have loaded
-// and processed already: they pass through LDS, with one barrier per row.
-// That needs every wavefront of the workgroup to have an item and to march
-// (the same rows, so the same barriers).  A halo column that is the strip's
-// own column (lane 0 of the first strip, lane 63 of the last, where the
-// halo index is clamped into the grid) takes the lane's own values.  Other
-// halo columns are loaded as before.
-struct EdgePlan {
-  bool lds = false;                            // the workgroup trades edges
-  bool nb_left = false, nb_right = false;      // neighbour strip in the group
-  bool own_left = false, own_right = false;    // halo column is the own one
-  int wave = 0;                                // wavefront in the group
+// A work item read with scalar loads (k is wave-uniform).
+__device__ __forceinline__ WorkItem scalar_item(const WorkItem* items, int k) {
+  return items[__builtin_amdgcn_readfirstlane(k)];
+}
+
+// The columns just outside a strip (its halo) reach the wavefront through a
+// ring of three row slots in LDS, per wavefront and side one value of each
+// traded plane.  A slot is filled when its row enters the window and read when
+// the row is used, so no register holds a halo value across rows.
+//
+// Where the values come from is decided per side:
+//  - the workgroup's W items are consecutive in the work list: horizontally
+//    adjacent strips of one segment (or of two, when a row has fewer than W
+//    strips).  A halo column is then the neighbour's edge column, which the
+//    neighbour has loaded and processed already and stores into this
+//    wavefront's ring, with one barrier per row.  That needs every wavefront
+//    of the workgroup to have an item and to march (the same rows, so the
+//    same barriers);
+//  - a halo column that is the strip's own column (the first strip's left, the
+//    last strip's right, where the halo index is clamped into the grid) is
+//    stored by the edge lane itself;
+//  - any other halo column is loaded from memory, one plane per lane: lanes
+//    0 .. P-1 load the left column's planes, lanes P .. 2P-1 the right one's,
+//    so a row's halo costs one load per field set.
+//
+// With the halo in registers (lanes 0 and 63 of one register per plane, field
+// set and row of the window) the FP64 kernels loaded 2P values per lane more
+// than they used, and two-component P needed 314 registers, one wavefront per
+// SIMD; now 256 and 5.  P (64 x 256^2, FP64) takes 110 us instead of 118, G
+// 134 instead of 139; 24 x 512^2 with two components 247 instead of 271 us and
+// 299 instead of 305; a film of 8 x 768^2 116 instead of 130 and 129 instead of
+// 135.  A mixed step of 64 x 256^2 with overlapping parts: 98.6 us, 105.5
+// before.  Reading the halo a row ahead of its use instead costs registers and
+// was slower (107 us).
+struct HaloPlan {
+  bool lds = false;            // the workgroup trades edges (barriers)
+  int dst_wave = -1;           // edge lanes: whose ring the own value goes to,
+  int dst_side = 0;            // and its side there (-1: nobody's)
+  bool mem[2] = {true, true};  // left, right column loaded from memory
+  int wave = 0;                // wavefront in the group
 };
 
 template <int W>
-__device__ __forceinline__ EdgePlan edge_plan(const StepArgs& a, const DevString& s,
-                                              const WorkItem& it) {
-  EdgePlan e;
+__device__ __forceinline__ HaloPlan halo_plan(const StepArgs& a, const DevString& s,
+                                              const WorkItem& it, const Strip& t) {
+  HaloPlan e;
   if constexpr (W > 1) {
+    e.wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     if (!a.edges) return e;
     const int groups = (a.nitems + W - 1) / W;
     const int kb = xcd_item(blockIdx.x, groups) * W;
     if (kb + W > a.nitems) return e;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     // Decided from the group's items alone, so every wavefront of the group
     // takes the same decision: all items march (they have bonds) over the
-    // same rows in the same direction (one segment of one image).
-    const WorkItem o0 = load_item(a.items, kb);
-    const int seg0 = o0.tile / s.tiles_x;
-    bool all = !(o0.flags & kItemNoBonds), left = false, right = false;
+    // same rows in the same direction (one segment of one image).  The items
+    // are read in one batch, ahead of any test of them.
+    WorkItem o[W];
+#pragma unroll
+    for (int q = 0; q < W; ++q) o[q] = scalar_item(a.items, kb + q);
+    const int first = o[0].tile - o[0].tile % s.tiles_x;  // the segment's first tile
+    int ok = 1, left = 0, right = 0;
 #pragma unroll
     for (int q = 0; q < W; ++q) {
-      const WorkItem o = q == 0 ? o0 : load_item(a.items, kb + q);
-      all = all && !(o.flags & kItemNoBonds) && o.string == o0.string && o.image == o0.image &&
-            o.tile / s.tiles_x == seg0;
-      left = left || (q == wave - 1 && o.tile == it.tile - 1);
-      right = right || (q == wave + 1 && o.tile == it.tile + 1);
+      ok &= (int)!(o[q].flags & kItemNoBonds) & (int)(o[q].string == o[0].string) &
+            (int)(o[q].image == o[0].image) & (int)(o[q].tile >= first) &
+            (int)(o[q].tile < first + s.tiles_x);
+      left |= (int)(q == e.wave - 1) & (int)(o[q].tile == it.tile - 1);
+      right |= (int)(q == e.wave + 1) & (int)(o[q].tile == it.tile + 1);
     }
+    const bool all = ok != 0;
     if (!all) return e;
     const int sx = it.tile % s.tiles_x;
+    const bool own_left = sx == 0, own_right = (sx + 1) * kTileX >= s.N;
+    const bool nb_left = !own_left && left, nb_right = !own_right && right;
     e.lds = true;
-    e.wave = wave;
-    e.own_left = sx == 0;
-    e.own_right = (sx + 1) * kTileX >= s.N;
-    e.nb_left = !e.own_left && left;
-    e.nb_right = !e.own_right && right;
+    e.mem[0] = !(own_left || nb_left);
+    e.mem[1] = !(own_right || nb_right);
+    if (t.lane == 0) {
+      e.dst_wave = nb_left ? e.wave - 1 : own_left ? e.wave : -1;
+      e.dst_side = nb_left ? 1 : 0;
+    } else if (t.lane == kWave - 1) {
+      e.dst_wave = nb_right ? e.wave + 1 : own_right ? e.wave : -1;
+      e.dst_side = nb_right ? 0 : 1;
+    }
   }
   return e;
 }
 
-// Whether this lane loads its halo column from memory.
-__device__ __forceinline__ bool halo_from_memory(const Strip& t, const EdgePlan& e) {
-  if (!t.edge) return false;
-  if (!e.lds) return true;
-  return t.lane == 0 ? !(e.nb_left || e.own_left) : !(e.nb_right || e.own_right);
+// The halo column this lane loads: its plane, whether its side comes from
+// memory, and the byte offset of (row 0, plane, column).  With a fixed A, a
+// load serves either the A planes or the psi planes; the lanes of the others
+// repeat an address that the load needs anyway.
+struct HaloLane {
+  int plane, side;
+  bool load;
+  unsigned off;    // fields, directions, gradients
+  unsigned off_a;  // the fixed A
+};
+template <class T, int P, bool NSF>
+__device__ __forceinline__ HaloLane halo_lane(const DevString& s, const Strip& t,
+                                              const HaloPlan& e) {
+  HaloLane h;
+  h.side = t.lane < P ? 0 : 1;
+  h.plane = t.lane - h.side * P;
+  h.load = t.lane < 2 * P && (h.side == 0 ? e.mem[0] : e.mem[1]);
+  const int x0 = t.i - t.lane;
+  const int col = h.side == 0 ? max(x0 - 1, 0) : min(x0 + kWave, s.N - 1);
+  const int ps = (int)s.plane_stride, psi = NSF ? max(h.plane, 2) : h.plane;
+  h.off = (unsigned)((psi * ps + col) * (int)sizeof(T));
+  h.off_a = (unsigned)((min(h.plane, 1) * ps + col) * (int)sizeof(T));
+  return h;
 }
 
 // The barrier of the edge exchange: LDS writes before it are visible to the
@@ -177,6 +231,42 @@ __device__ __forceinline__ void edge_barrier() {
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt and expcnt left as they are
   __builtin_amdgcn_s_barrier();
   memory_fence_compiler();
+}
+
+// The raw loads of a row: own columns of x and d, and this lane's halo value
+// of each (HaloLane).
+template <class T, int NC>
+struct GBatch {
+  static constexpr int P = 2 + 2 * NC;
+  T x[P], d[P], hx, hd, ha;
+  uint16_t nn;
+};
+
+// A row of the window: A with its x-neighbours, and psi.
+template <class T, int NC>
+struct GWin {
+  T ax, ay, axl, axr, ayl, ayr;
+  T u[NC], v[NC];
+  uint16_t nn;
+};
+
+template <class T, int NC, bool UPD, bool NSF>
+__device__ __forceinline__ void g_batch(GBatch<T, NC>& r, const GBufs& b, int row, int P_,
+                                        const Strip& t, const HaloLane& h) {
+  const unsigned o = (unsigned)((row * P_ + t.ic) * (int)sizeof(T));
+#pragma unroll
+  for (int p = 0; p < GBatch<T, NC>::P; ++p) {
+    r.x[p] = bload<T>(p < 2 ? b.xa : b.x, o, p * b.ps);
+    r.d[p] = (UPD && !(NSF && p < 2)) ? bload<T>(b.d, o, p * b.ps) : (T)0;
+  }
+  r.hx = r.hd = r.ha = (T)0;
+  if (h.load) {
+    const unsigned ro = (unsigned)(row * P_ * (int)sizeof(T)), ho = h.off + ro;
+    r.hx = bload<T>(b.x, ho, 0);
+    if (UPD) r.hd = bload<T>(b.d, ho, 0);
+    if (NSF) r.ha = bload<T>(b.xa, h.off_a + ro, 0);  // the fixed A, maybe image 0's
+  }
+  r.nn = bload_u16(b.nn, (unsigned)((row * P_ + t.ic) * (int)sizeof(uint16_t)));
 }
 
 template <class T, int NC, bool UPD, bool NSF, bool PL, bool MW>
@@ -209,63 +299,46 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
   gptr<const double> __restrict__ hp = as_global(s.h.p);
   const T hv = (T)s.h.v;
   double acc_s[2] = {0, 0}, acc_c[2] = {0, 0};
-  auto nnoff = [&](int row) { return (unsigned)((row * P_ + t.ic) * (int)sizeof(uint16_t)); };
-  // Edge exchange (EdgePlan): in mixed precision a row's A values outside
-  // the strip are final only once the neighbours' edges are in, so A's
-  // x-neighbours are formed one row later (g_finish), when the row becomes
-  // the next row of the march.
   constexpr int W = step_waves<T>();
-  const EdgePlan ep = edge_plan<W>(a, s, it);
-  const bool hmem = halo_from_memory(t, ep);
-  constexpr int EV = 2 + 2 * NC;  // A and psi
-  __shared__ T edges[W > 1 ? 3 : 1][W][2][EV];
-  auto put_edges = [&](const GRow<T, NC>& w, auto slot_tag) {
+  constexpr int EV = 2 + 2 * NC;  // traded values of a row: A and psi
+  const HaloPlan hp_ = halo_plan<W>(a, s, it, t);
+  const HaloLane hl = halo_lane<T, EV, NSF>(s, t, hp_);
+  __shared__ T ring[W][3][2][EV];
+  // A row's raw loads into window values and its slot of the ring.
+  auto process = [&](GWin<T, NC>& w, const GBatch<T, NC>& r, auto slot_tag) {
     constexpr int SL = decltype(slot_tag)::value;
-    if constexpr (W > 1) {
-      if (ep.lds && t.edge) {
-        T* dst = edges[SL][ep.wave][t.lane == 0 ? 0 : 1];
-        dst[0] = w.ax;
-        dst[1] = w.ay;
+    T c[EV];
 #pragma unroll
-        for (int q = 0; q < NC; ++q) {
-          dst[2 + 2 * q] = w.u[q];
-          dst[3 + 2 * q] = w.v[q];
-        }
+    for (int p = 0; p < EV; ++p) c[p] = UPD ? fma(al, r.d[p], r.x[p]) : r.x[p];
+    T e = UPD ? fma(al, r.hd, r.hx) : r.hx;
+    if (NSF) e = hl.plane < 2 ? r.ha : e;  // the fixed A takes no update
+    w.ax = c[PAX];
+    w.ay = c[PAY];
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      w.u[q] = c[PU1 + 2 * q];
+      w.v[q] = c[PV1 + 2 * q];
+    }
+    w.nn = r.nn;
+    if (hl.load) ring[hp_.wave][SL][hl.side][hl.plane] = e;
+    if constexpr (W > 1) {
+      if (hp_.dst_wave >= 0) {
+        T* dst = ring[hp_.dst_wave][SL][hp_.dst_side];
+#pragma unroll
+        for (int p = 0; p < EV; ++p) dst[p] = c[p];
       }
     }
   };
-  auto finish = [&](GRow<T, NC>& w, auto slot_tag) {
-    constexpr int SL = decltype(slot_tag)::value;
-    if constexpr (W > 1) {
-      if (ep.lds && t.edge) {
-        const bool left = t.lane == 0;
-        if (left ? ep.nb_left : ep.nb_right) {
-          const T* src = edges[SL][left ? ep.wave - 1 : ep.wave + 1][left ? 1 : 0];
-          w.eax = src[0];
-          w.eay = src[1];
-#pragma unroll
-          for (int q = 0; q < NC; ++q) {
-            w.eu[q] = src[2 + 2 * q];
-            w.ev[q] = src[3 + 2 * q];
-          }
-        } else if (left ? ep.own_left : ep.own_right) {
-          w.eax = w.ax;
-          w.eay = w.ay;
-#pragma unroll
-          for (int q = 0; q < NC; ++q) {
-            w.eu[q] = w.u[q];
-            w.ev[q] = w.v[q];
-          }
-        }
-      }
-      g_finish<T, NC>(w);
-    }
-  };
-  auto process = [&](GRow<T, NC>& w, const GRaw<T, NC>& r) {
-    if constexpr (W > 1)
-      g_process_own<T, NC>(w, r, al, UPD);
-    else
-      g_process<T, NC>(w, r, al, UPD);
+  // This side's halo value of a plane of the row in a slot.
+  const int side = t.lane == kWave - 1 ? 1 : 0;
+  auto edge = [&](auto slot_tag, int p) { return ring[hp_.wave][decltype(slot_tag)::value][side][p]; };
+  // A's x-neighbours of a row, once its slot is filled.
+  auto finish = [&](GWin<T, NC>& w, auto slot_tag) {
+    const T ex = edge(slot_tag, PAX), ey = edge(slot_tag, PAY);
+    w.axl = from_left(w.ax, ex);
+    w.axr = from_right(w.ax, ex);
+    w.ayl = from_left(w.ay, ey);
+    w.ayr = from_right(w.ay, ey);
   };
 
   // The march is the only part that depends on the direction
@@ -314,7 +387,7 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
     for (int j = t.j0; j < t.j1; ++j) {
       const unsigned o = (unsigned)((j * P_ + t.ic) * (int)sizeof(T));
 #pragma unroll
-      for (int p = P0; p < GRaw<T, NC>::P; ++p)
+      for (int p = P0; p < EV; ++p)
         bstore(bload<T>(b.x, o, p * b.ps), b.xo, o, p * b.ps);
     }
   };
@@ -330,21 +403,18 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
     // when UP, up (rows j1-1 .. j0); the previous row of the march is then
     // row j + 1.
     const int jb = UP ? t.j1 - 1 : t.j0;  // first row of the march
-    GRaw<T, NC> raw;
-    GRow<T, NC> w[3];
+    GBatch<T, NC> raw;
+    GWin<T, NC> w[3];
     GSide<T, NC, PL> sd[3];
-    g_load<T, NC, UPD, NSF>(raw, b, clampr(jb - D, N), P_, t, nnoff(clampr(jb - D, N)), hmem);
-    process(w[0], raw);
-    g_load<T, NC, UPD, NSF>(raw, b, clampr(jb, N), P_, t, nnoff(clampr(jb, N)), hmem);
-    process(w[1], raw);
-    g_load<T, NC, UPD, NSF>(raw, b, clampr(jb + D, N), P_, t, nnoff(clampr(jb + D, N)), hmem);
-    process(w[2], raw);
+    g_batch<T, NC, UPD, NSF>(raw, b, clampr(jb - D, N), P_, t, hl);
+    process(w[0], raw, S0());
+    g_batch<T, NC, UPD, NSF>(raw, b, clampr(jb, N), P_, t, hl);
+    process(w[1], raw, S1());
+    g_batch<T, NC, UPD, NSF>(raw, b, clampr(jb + D, N), P_, t, hl);
+    process(w[2], raw, S2());
     g_side_load<T, NC, NSF, PL, MW>(sd[1], b, jb, P_, t, pv, hp, N);
-    // The first rows' edges; row jb + D is finished at the first row's start.
-    put_edges(w[0], S0());
-    put_edges(w[1], S1());
-    put_edges(w[2], S2());
-    if (ep.lds) edge_barrier();
+    // Row jb + D is finished at the first row's start.
+    if (hp_.lds) edge_barrier();
     finish(w[0], S0());
     finish(w[1], S1());
 
@@ -359,17 +429,17 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
       constexpr int IP = decltype(ip_tag)::value, IC = decltype(ic_tag)::value;
       constexpr int IN = decltype(in_tag)::value;
       constexpr bool BATCH = decltype(batch_tag)::value;
-      GRow<T, NC>& wm = w[UP ? IN : IP];  // row j - 1
-      GRow<T, NC>& wc = w[IC];
-      GRow<T, NC>& wpl = w[UP ? IP : IN];  // row j + 1
+      GWin<T, NC>& wm = w[UP ? IN : IP];  // row j - 1
+      GWin<T, NC>& wc = w[IC];
+      GWin<T, NC>& wpl = w[UP ? IP : IN];  // row j + 1
       const bool live = store && (UP ? j >= t.j0 : j < t.j1);
       if constexpr (BATCH) {
-        g_load<T, NC, UPD, NSF>(raw, b, clampr(j + 2 * D, N), P_, t,
-                                nnoff(clampr(j + 2 * D, N)), hmem);
+        g_batch<T, NC, UPD, NSF>(raw, b, clampr(j + 2 * D, N), P_, t, hl);
         g_side_load<T, NC, NSF, PL, MW>(sd[IN], b, clampr(j + D, N), P_, t, pv, hp, N);
       }
-      // Row j + D, processed one row ago, takes its neighbours' edges.
-      if (ep.lds) edge_barrier();
+      // Row j + D, processed one row ago, takes its halo; row j's slot is as
+      // full.
+      if (hp_.lds) edge_barrier();
       finish(w[IN], in_tag);
       __builtin_amdgcn_sched_barrier(0);
 
@@ -384,10 +454,11 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
       for (int q = 0; q < NC; ++q) {
         nb.u[q][0] = wc.u[q];
         nb.v[q][0] = wc.v[q];
-        nb.u[q][1] = from_right(wc.u[q], wc.eu[q]);
-        nb.v[q][1] = from_right(wc.v[q], wc.ev[q]);
-        nb.u[q][2] = from_left(wc.u[q], wc.eu[q]);
-        nb.v[q][2] = from_left(wc.v[q], wc.ev[q]);
+        const T eu = edge(ic_tag, PU1 + 2 * q), ev = edge(ic_tag, PV1 + 2 * q);
+        nb.u[q][1] = from_right(wc.u[q], eu);
+        nb.v[q][1] = from_right(wc.v[q], ev);
+        nb.u[q][2] = from_left(wc.u[q], eu);
+        nb.v[q][2] = from_left(wc.v[q], ev);
         nb.u[q][3] = wpl.u[q];
         nb.v[q][3] = wpl.v[q];
         nb.u[q][4] = wm.u[q];
@@ -443,12 +514,10 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
       }
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (BATCH) {
-        process(w[IP], raw);
-        put_edges(w[IP], ip_tag);
-        if constexpr (W > 1)
-          pin_row_own<T, NC>(w[IP]);
-        else
-          pin_row<T, NC>(w[IP]);
+        process(w[IP], raw, ip_tag);
+        pin(w[IP].ax), pin(w[IP].ay), pin(w[IP].nn);
+#pragma unroll
+        for (int q = 0; q < NC; ++q) pin(w[IP].u[q]), pin(w[IP].v[q]);
         pin_side<T, NC, PL>(sd[IN]);
         memory_fence_compiler();
       }
@@ -507,25 +576,24 @@ template <class T, int NC, bool UPD, bool NSF, bool PL, bool MW>
 __global__ __launch_bounds__(kWave * step_waves<T>()) void k_grad(StepArgs a) {
   const int k = step_item<step_waves<T>()>(a.nitems);
   if (k >= a.nitems) return;
-  const WorkItem it = load_item(a.items, k);
+  const WorkItem it = scalar_item(a.items, k);
   grad_body<T, NC, UPD, NSF, PL, MW>(a, a.strings[it.string], it);
 }
 
 // ---------------------------------------------------------------------------
 // P kernel.
+// The raw loads of a row, with this lane's halo value of each field set.
 template <class T, int NC>
 struct PRaw {
   static constexpr int P = 2 + 2 * NC;
-  T x[P], g[P], d[P], hx[P], hg[P], hd[P];
+  T x[P], g[P], d[P], hx, hg, hd, ha;
   uint16_t nn;
 };
 
 template <class T, int NC>
 struct PRow {
   T ax, ay, dax, day;              // A and its new direction
-  T eax, eay, edax, eday;          // the same outside the strip (lanes 0 / 63)
   T u[NC], v[NC], du[NC], dv[NC];  // psi and its new direction
-  T eu[NC], ev[NC], edu[NC], edv[NC];
   uint16_t nn;
 };
 
@@ -536,121 +604,32 @@ struct PBufs {
 
 template <class T, int NC, bool NSF>
 __device__ __forceinline__ void p_load(PRaw<T, NC>& r, const PBufs& b, int row, int P_,
-                                       const Strip& t, unsigned nnoff, bool halo) {
-  const RowOff o = row_off<T>(row, P_, t);
+                                       const Strip& t, const HaloLane& h) {
+  const unsigned o = (unsigned)((row * P_ + t.ic) * (int)sizeof(T));
 #pragma unroll
   for (int p = 0; p < PRaw<T, NC>::P; ++p) {
     const bool dir = !(NSF && p < 2);
-    r.x[p] = bload<T>(p < 2 ? b.xa : b.x, o.own, p * b.ps);
-    r.g[p] = dir ? bload<T>(b.g, o.own, p * b.ps) : (T)0;
-    r.d[p] = dir ? bload<T>(b.d, o.own, p * b.ps) : (T)0;
+    r.x[p] = bload<T>(p < 2 ? b.xa : b.x, o, p * b.ps);
+    r.g[p] = dir ? bload<T>(b.g, o, p * b.ps) : (T)0;
+    r.d[p] = dir ? bload<T>(b.d, o, p * b.ps) : (T)0;
   }
-#pragma unroll
-  for (int p = 0; p < PRaw<T, NC>::P; ++p) r.hx[p] = r.hg[p] = r.hd[p] = (T)0;
-  if (halo) {
-#pragma unroll
-    for (int p = 0; p < PRaw<T, NC>::P; ++p) {
-      const bool dir = !(NSF && p < 2);
-      r.hx[p] = bload<T>(p < 2 ? b.xa : b.x, o.halo, p * b.ps);
-      r.hg[p] = dir ? bload<T>(b.g, o.halo, p * b.ps) : (T)0;
-      r.hd[p] = dir ? bload<T>(b.d, o.halo, p * b.ps) : (T)0;
-    }
+  r.hx = r.hg = r.hd = r.ha = (T)0;
+  if (h.load) {
+    const unsigned ro = (unsigned)(row * P_ * (int)sizeof(T)), ho = h.off + ro;
+    r.hx = bload<T>(b.x, ho, 0);
+    r.hg = bload<T>(b.g, ho, 0);
+    r.hd = bload<T>(b.d, ho, 0);
+    if (NSF) r.ha = bload<T>(b.xa, h.off_a + ro, 0);  // the fixed A, maybe image 0's
   }
-  r.nn = bload_u16(b.nn, nnoff);
+  r.nn = bload_u16(b.nn, (unsigned)((row * P_ + t.ic) * (int)sizeof(uint16_t)));
 }
 
-// d = -g + beta d  (computeStepDirection, nlcg.cu:985-993)
 template <class T, int NC>
 __device__ __forceinline__ void pin_row(PRow<T, NC>& w) {
-  pin(w.ax), pin(w.ay), pin(w.dax), pin(w.day), pin(w.eax), pin(w.eay), pin(w.edax), pin(w.eday);
+  pin(w.ax), pin(w.ay), pin(w.dax), pin(w.day);
 #pragma unroll
-  for (int q = 0; q < NC; ++q) {
-    pin(w.u[q]), pin(w.v[q]), pin(w.du[q]), pin(w.dv[q]);
-    pin(w.eu[q]), pin(w.ev[q]), pin(w.edu[q]), pin(w.edv[q]);
-  }
+  for (int q = 0; q < NC; ++q) pin(w.u[q]), pin(w.v[q]), pin(w.du[q]), pin(w.dv[q]);
   pin(w.nn);
-}
-
-template <class T, int NC>
-__device__ __forceinline__ void p_process(PRow<T, NC>& w, const PRaw<T, NC>& r, T beta) {
-  T dn[PRaw<T, NC>::P], en[PRaw<T, NC>::P];
-#pragma unroll
-  for (int p = 0; p < PRaw<T, NC>::P; ++p) {
-    dn[p] = fma(beta, r.d[p], -r.g[p]);
-    en[p] = fma(beta, r.hd[p], -r.hg[p]);
-  }
-  w.ax = r.x[PAX];
-  w.ay = r.x[PAY];
-  w.eax = r.hx[PAX];
-  w.eay = r.hx[PAY];
-  w.dax = dn[PAX];
-  w.day = dn[PAY];
-  w.edax = en[PAX];
-  w.eday = en[PAY];
-#pragma unroll
-  for (int q = 0; q < NC; ++q) {
-    w.u[q] = r.x[PU1 + 2 * q];
-    w.v[q] = r.x[PV1 + 2 * q];
-    w.eu[q] = r.hx[PU1 + 2 * q];
-    w.ev[q] = r.hx[PV1 + 2 * q];
-    w.du[q] = dn[PU1 + 2 * q];
-    w.dv[q] = dn[PV1 + 2 * q];
-    w.edu[q] = en[PU1 + 2 * q];
-    w.edv[q] = en[PV1 + 2 * q];
-  }
-  w.nn = r.nn;
-}
-
-// A P row's values traded at the strip edges: A, its new direction, psi and
-// its new direction.
-template <int NC>
-constexpr int p_edge_values() {
-  return 4 + 4 * NC;
-}
-
-template <class T, int NC>
-__device__ __forceinline__ void p_put_edges(const PRow<T, NC>& w, T* dst) {
-  dst[0] = w.ax;
-  dst[1] = w.ay;
-  dst[2] = w.dax;
-  dst[3] = w.day;
-#pragma unroll
-  for (int q = 0; q < NC; ++q) {
-    dst[4 + 4 * q] = w.u[q];
-    dst[5 + 4 * q] = w.v[q];
-    dst[6 + 4 * q] = w.du[q];
-    dst[7 + 4 * q] = w.dv[q];
-  }
-}
-
-template <class T, int NC>
-__device__ __forceinline__ void p_get_edges(PRow<T, NC>& w, const T* src) {
-  w.eax = src[0];
-  w.eay = src[1];
-  w.edax = src[2];
-  w.eday = src[3];
-#pragma unroll
-  for (int q = 0; q < NC; ++q) {
-    w.eu[q] = src[4 + 4 * q];
-    w.ev[q] = src[5 + 4 * q];
-    w.edu[q] = src[6 + 4 * q];
-    w.edv[q] = src[7 + 4 * q];
-  }
-}
-
-template <class T, int NC>
-__device__ __forceinline__ void p_own_edges(PRow<T, NC>& w) {
-  w.eax = w.ax;
-  w.eay = w.ay;
-  w.edax = w.dax;
-  w.eday = w.day;
-#pragma unroll
-  for (int q = 0; q < NC; ++q) {
-    w.eu[q] = w.u[q];
-    w.ev[q] = w.v[q];
-    w.edu[q] = w.du[q];
-    w.edv[q] = w.dv[q];
-  }
 }
 
 template <class T, int NC, bool NSF, bool PL>
@@ -671,8 +650,7 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
   // The Polak-Ribiere beta (computeStepDirection, nlcg.cu:972-982): every
   // wavefront totals the gradient kernel's partials of its image in the same
   // fixed order, so all of them hold the same beta.  The old norm read here
-  // sits in the other slot than the one the image's first tile stores at the
-  // end of the body.
+  // sits in the other slot than the one the image's first tile stores.
   ImageScalars* const scp = a.sc + s.img0 + t.n;
   auto totals = [&](double& gnorm2, double& gdelta, double& beta_d) {
     double fin[2];
@@ -681,40 +659,20 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
     gdelta = fin[1];
     beta_d = a.nlcg ? fmax(gdelta / scp->g_norm2[a.sold], 0.0) : 0.0;
   };
-  auto nnoff = [&](int row) { return (unsigned)((row * P_ + t.ic) * (int)sizeof(uint16_t)); };
   constexpr int W = step_waves<T>();
-  const EdgePlan ep = edge_plan<W>(a, s, it);
-  const bool hmem = halo_from_memory(t, ep);
-  // Edge values per row slot of the window, wavefront and side (lane 0,
-  // lane 63).
-  constexpr int EV = p_edge_values<NC>();
-  __shared__ T edges[W > 1 ? 3 : 1][W][2][EV];
-  auto put_edges = [&](const PRow<T, NC>& w, auto slot_tag) {
-    constexpr int SL = decltype(slot_tag)::value;
-    if constexpr (W > 1) {
-      if (ep.lds && t.edge) p_put_edges<T, NC>(w, edges[SL][ep.wave][t.lane == 0 ? 0 : 1]);
-    }
-  };
-  auto get_edges = [&](PRow<T, NC>& w, auto slot_tag) {
-    constexpr int SL = decltype(slot_tag)::value;
-    if constexpr (W > 1) {
-      if (ep.lds && t.edge) {
-        const bool left = t.lane == 0;
-        if (left ? ep.nb_left : ep.nb_right)
-          p_get_edges<T, NC>(w, edges[SL][left ? ep.wave - 1 : ep.wave + 1][left ? 1 : 0]);
-        else if (left ? ep.own_left : ep.own_right)
-          p_own_edges<T, NC>(w);
-      }
-    }
-  };
+  constexpr int P = PRaw<T, NC>::P;
+  const HaloPlan hp_ = halo_plan<W>(a, s, it, t);
+  const HaloLane hl = halo_lane<T, P, NSF>(s, t, hp_);
+  // x and the new direction of every plane.
+  __shared__ T ring[W][3][2][2][P];
   // The march is the only part that depends on the direction
   // (marches_up).  Its rows are loaded after beta is totalled: holding a row
   // across the partials' reduction costs the mixed kernels a wave per SIMD
   // (129 VGPRs), more than the overlap gains.
   const bool up = marches_up(s, it);
   const bool bonds = !(it.flags & kItemNoBonds);
-  double gnorm2, gdelta, beta_d;
-  totals(gnorm2, gdelta, beta_d);
+  double gnorm2 = 0, gdelta = 0, beta_d = 0;
+  if (bonds || it.tile == 0) totals(gnorm2, gdelta, beta_d);
   const T beta = uniform_value((T)beta_d);
   constexpr bool nsf = NSF;
   const bool exact = s.poly_exact;
@@ -736,7 +694,16 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
   const T hv = (T)s.h.v * dx;
   double acc_s[5] = {0, 0, 0, 0, 0}, acc_c[5] = {0, 0, 0, 0, 0};
   // Everything the march needs from the string's descriptor is read above,
-  // before the branch and before any store, so it stays in scalar registers.
+  // before the branch and before the first store, so it stays in scalar
+  // registers.
+  if (it.tile == 0 && lane_id() == 0) {
+    scp->g_norm2[a.scur] = gnorm2;
+    scp->g_delta_g = gdelta;
+    scp->beta = beta_d;
+    // A gradient total that is not finite (NaN or +-Inf) marks the step;
+    // the host reads the flag once per outer iteration.
+    if (!__builtin_isfinite(gnorm2) || !__builtin_isfinite(gdelta)) *a.health = 1;
+  }
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
   using S2 = std::integral_constant<int, 2>;
@@ -751,20 +718,58 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
     PRaw<T, NC> raw;
     PRow<T, NC> w[3];
     RowParams<T, NC, PL> rp[3];
-    p_load<T, NC, NSF>(raw, b, clampr(jb - D, N), P_, t, nnoff(clampr(jb - D, N)), hmem);
-    p_process<T, NC>(w[0], raw, beta);
-    p_load<T, NC, NSF>(raw, b, clampr(jb, N), P_, t, nnoff(clampr(jb, N)), hmem);
-    p_process<T, NC>(w[1], raw, beta);
-    p_load<T, NC, NSF>(raw, b, clampr(jb + D, N), P_, t, nnoff(clampr(jb + D, N)), hmem);
-    p_process<T, NC>(w[2], raw, beta);
+    // A row's raw loads into window values, d = -g + beta d
+    // (computeStepDirection, nlcg.cu:985-993), and its slot of the ring.
+    auto process = [&](PRow<T, NC>& w, const PRaw<T, NC>& r, auto slot_tag) {
+      constexpr int SL = decltype(slot_tag)::value;
+      T dn[P];
+#pragma unroll
+      for (int p = 0; p < P; ++p) dn[p] = fma(beta, r.d[p], -r.g[p]);
+      T ex = r.hx, en = fma(beta, r.hd, -r.hg);
+      if (NSF) {  // the fixed A, with no direction
+        ex = hl.plane < 2 ? r.ha : ex;
+        en = hl.plane < 2 ? (T)0 : en;
+      }
+      w.ax = r.x[PAX];
+      w.ay = r.x[PAY];
+      w.dax = dn[PAX];
+      w.day = dn[PAY];
+#pragma unroll
+      for (int q = 0; q < NC; ++q) {
+        w.u[q] = r.x[PU1 + 2 * q];
+        w.v[q] = r.x[PV1 + 2 * q];
+        w.du[q] = dn[PU1 + 2 * q];
+        w.dv[q] = dn[PV1 + 2 * q];
+      }
+      w.nn = r.nn;
+      if (hl.load) {
+        ring[hp_.wave][SL][hl.side][0][hl.plane] = ex;
+        ring[hp_.wave][SL][hl.side][1][hl.plane] = en;
+      }
+      if constexpr (W > 1) {
+        if (hp_.dst_wave >= 0) {
+          T(*dst)[P] = ring[hp_.dst_wave][SL][hp_.dst_side];
+#pragma unroll
+          for (int p = 0; p < P; ++p) {
+            dst[0][p] = r.x[p];
+            dst[1][p] = dn[p];
+          }
+        }
+      }
+    };
+    // This side's halo value of plane p of x (set 0) or the new direction
+    // (set 1), of the row in a slot.
+    const int side = t.lane == kWave - 1 ? 1 : 0;
+    auto edge = [&](auto slot_tag, int set, int p) {
+      return ring[hp_.wave][decltype(slot_tag)::value][side][set][p];
+    };
+    p_load<T, NC, NSF>(raw, b, clampr(jb - D, N), P_, t, hl);
+    process(w[0], raw, S0());
+    p_load<T, NC, NSF>(raw, b, clampr(jb, N), P_, t, hl);
+    process(w[1], raw, S1());
+    p_load<T, NC, NSF>(raw, b, clampr(jb + D, N), P_, t, hl);
+    process(w[2], raw, S2());
     rp[1].load(pv, hp, (long long)jb * P_ + t.ic, jb, N, P_, t);
-    // The first rows' edges; row jb + D's are read at the first row's start.
-    put_edges(w[0], S0());
-    put_edges(w[1], S1());
-    put_edges(w[2], S2());
-    if (ep.lds) edge_barrier();
-    get_edges(w[0], S0());
-    get_edges(w[1], S1());
 
     // Row j: one batch of loads (the fields of row j + 2D, the parameters of
     // row j + D), the quartic of row j from registers, the batch into the
@@ -778,36 +783,34 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
       PRow<T, NC>& wpl = w[UP ? IP : IN];  // row j + 1
       const bool live = store && (UP ? j >= t.j0 : j < t.j1);
       if constexpr (BATCH) {
-        p_load<T, NC, NSF>(raw, b, clampr(j + 2 * D, N), P_, t, nnoff(clampr(j + 2 * D, N)),
-                           hmem);
+        p_load<T, NC, NSF>(raw, b, clampr(j + 2 * D, N), P_, t, hl);
         const int r1 = clampr(j + D, N);
         rp[IN].load(pv, hp, (long long)r1 * P_ + t.ic, r1, N, P_, t);
       }
-      // Row j + D's edges, stored by the neighbours when they processed it
-      // one row ago: row j + D is the current row at the next row.
-      if (ep.lds) edge_barrier();
-      get_edges(w[IN], in_tag);
+      // The neighbours' edges of row j, stored when they processed it, and
+      // before row j + 2D's take the slot of row j - D.
+      if (hp_.lds) edge_barrier();
       __builtin_amdgcn_sched_barrier(0);
 
       PolyNbhd<T, NC> nb;
       nb.ax[0] = wc.ax;
-      nb.ax[1] = from_right(wc.ax, wc.eax);
+      nb.ax[1] = from_right(wc.ax, edge(ic_tag, 0, PAX));
       nb.ax[2] = 0;
       nb.ax[3] = wpl.ax;
       nb.ax[4] = wm.ax;
       nb.ay[0] = wc.ay;
-      nb.ay[1] = from_right(wc.ay, wc.eay);
-      nb.ay[2] = from_left(wc.ay, wc.eay);
+      nb.ay[1] = from_right(wc.ay, edge(ic_tag, 0, PAY));
+      nb.ay[2] = from_left(wc.ay, edge(ic_tag, 0, PAY));
       nb.ay[3] = wpl.ay;
       nb.ay[4] = 0;
       nb.dax[0] = wc.dax;
-      nb.dax[1] = from_right(wc.dax, wc.edax);
+      nb.dax[1] = from_right(wc.dax, edge(ic_tag, 1, PAX));
       nb.dax[2] = 0;
       nb.dax[3] = wpl.dax;
       nb.dax[4] = wm.dax;
       nb.day[0] = wc.day;
-      nb.day[1] = from_right(wc.day, wc.eday);
-      nb.day[2] = from_left(wc.day, wc.eday);
+      nb.day[1] = from_right(wc.day, edge(ic_tag, 1, PAY));
+      nb.day[2] = from_left(wc.day, edge(ic_tag, 1, PAY));
       nb.day[3] = wpl.day;
       nb.day[4] = 0;
 #pragma unroll
@@ -816,10 +819,10 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
         nb.v[q][0] = wc.v[q];
         nb.du[q][0] = wc.du[q];
         nb.dv[q][0] = wc.dv[q];
-        nb.u[q][1] = from_right(wc.u[q], wc.eu[q]);
-        nb.v[q][1] = from_right(wc.v[q], wc.ev[q]);
-        nb.du[q][1] = from_right(wc.du[q], wc.edu[q]);
-        nb.dv[q][1] = from_right(wc.dv[q], wc.edv[q]);
+        nb.u[q][1] = from_right(wc.u[q], edge(ic_tag, 0, PU1 + 2 * q));
+        nb.v[q][1] = from_right(wc.v[q], edge(ic_tag, 0, PV1 + 2 * q));
+        nb.du[q][1] = from_right(wc.du[q], edge(ic_tag, 1, PU1 + 2 * q));
+        nb.dv[q][1] = from_right(wc.dv[q], edge(ic_tag, 1, PV1 + 2 * q));
         nb.u[q][2] = wpl.u[q];
         nb.v[q][2] = wpl.v[q];
         nb.du[q][2] = wpl.du[q];
@@ -842,8 +845,7 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
       }
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (BATCH) {
-        p_process<T, NC>(w[IP], raw, beta);
-        put_edges(w[IP], ip_tag);
+        process(w[IP], raw, ip_tag);
         pin_row<T, NC>(w[IP]);
         if constexpr (PL) {
 #pragma unroll
@@ -889,28 +891,13 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
   }
 
   publish_partial<5, COMP>(acc_s, acc_c, s.part_p, t.n, t.tile, s.tiles_x * s.tiles_y);
-  // The first tile's wavefront recomputes the totals here (same order, same
-  // values) rather than keeping them in registers across the march, and
-  // stores them only now: a store before the march would make the compiler
-  // read the descriptor with vector loads.
-  if (it.tile == 0) {
-    totals(gnorm2, gdelta, beta_d);
-    if (lane_id() == 0) {
-      scp->g_norm2[a.scur] = gnorm2;
-      scp->g_delta_g = gdelta;
-      scp->beta = beta_d;
-      // A gradient total that is not finite (NaN or +-Inf) marks the step;
-      // the host reads the flag once per outer iteration.
-      if (!__builtin_isfinite(gnorm2) || !__builtin_isfinite(gdelta)) *a.health = 1;
-    }
-  }
 }
 
 template <class T, int NC, bool NSF, bool PL>
 __global__ __launch_bounds__(kWave * step_waves<T>()) void k_poly(StepArgs a) {
   const int k = step_item<step_waves<T>()>(a.nitems);
   if (k >= a.nitems) return;
-  const WorkItem it = load_item(a.items, k);
+  const WorkItem it = scalar_item(a.items, k);
   poly_body<T, NC, NSF, PL>(a, a.strings[it.string], it);
 }
 
