@@ -317,7 +317,7 @@ int run_aux(mepgl_ctx* c, const AuxArgs& a, int which, int arg) {
     if (int rc = settle_ls(c)) return rc;
   }
   if (c->dry) return MEPGL_OK;
-  if (which == kKernelArclen) {
+  if (which == kKernelArclen || which == kKernelEnergy) {
     // Launched once per item class, like the step kernels.
     for (const auto& g : c->groups) {
       AuxArgs ag = a;

@@ -67,7 +67,7 @@ struct AuxArgs {
   double* out;          // per global image (energy)
   double* const* jb;    // per string JB planes (device array of pointers)
   int only_string;      // scalar maintenance: string index, or -1 for all
-  int nc, pl;           // arclength: class of every item in `items`
+  int nc, pl;           // arclength, energy: class of every item in `items`
                         // (components, parameter planes)
 };
 

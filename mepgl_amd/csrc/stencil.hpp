@@ -486,54 +486,62 @@ __device__ __forceinline__ Quartic<T> site_poly(const PolyNbhd<T, NC>& s,
 
 // ---------------------------------------------------------------------------
 // Energy density of one site in double, freeEnergyDensity nlcg.cu:105-214.
+// The fused operations are written out and the compiler forms no others, so
+// every kernel that evaluates a site gets the same bits.
 template <int NC>
 __device__ __forceinline__ double site_energy(const PolyNbhd<double, NC>& s,
                                               const CompConst<double> (&k)[NC], double eta,
                                               double gamma, double delta, double idx,
                                               double dx2, int sc, int cm, bool nsf) {
+#pragma clang fp contract(off)
   const double af = quad_count(sc) * 0.25;
   double nl = 0;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const double u = s.u[c][0], v = s.v[c][0];
-    nl += 0.5 * k[c].b * sq(k[c].ab + u * u + v * v);
+    const double n0 = fma(v, v, fma(u, u, k[c].ab));
+    nl = fma((0.5 * k[c].b) * n0, n0, nl);
   }
   if (NC == 2) {
     const double u1 = s.u[0][0], v1 = s.v[0][0], u2 = s.u[NC - 1][0], v2 = s.v[NC - 1][0];
-    nl += eta * (u1 * u2 + v1 * v2);
-    nl += gamma * 0.5 * (u1 * u1 + v1 * v1) * (u2 * u2 + v2 * v2);
-    nl += delta * 0.5 * (sq(u1 * u2 + v1 * v2) - sq(u1 * v2 - v1 * u2));
+    const double P = fma(v1, v2, u1 * u2), Q = fma(-v1, u2, u1 * v2);
+    nl = fma(eta, P, nl);
+    nl = fma((gamma * 0.5) * fma(v1, v1, u1 * u1), fma(v2, v2, u2 * u2), nl);
+    nl = fma(delta * 0.5, fma(P, P, -(Q * Q)), nl);
   }
   nl *= af;
-  double kx = 0, ky = 0;
+  // One kinetic bond: the sum of the squares at both of its ends.
+  auto bond = [&](double u0, double v0, double A0, double un, double vn, double An, double q) {
+#pragma clang fp contract(off)
+    const double Du = (un - u0) * idx, Dv = (vn - v0) * idx, q0 = q * A0, qn = q * An;
+    const double t1 = fma(q0, v0, Du), t2 = fma(qn, vn, Du);
+    const double t3 = fma(-q0, u0, Dv), t4 = fma(-qn, un, Dv);
+    return fma(t4, t4, fma(t3, t3, fma(t2, t2, t1 * t1)));
+  };
+  // An absent bond (bits 0 and 2) has weight 0.
+  const unsigned sp = pair_bits(sc);
+  const double wx = bitof(sc, 0) ? wx_fwd(sp) * 0.25 : 0.0;
+  const double wy = bitof(sc, 2) ? wy_fwd(sp) * 0.25 : 0.0;
+  double e = nl;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const double q = k[c].q;
-    if (bitof(sc, 0)) {
-      const double Du = (s.u[c][1] - s.u[c][0]) * idx, Dv = (s.v[c][1] - s.v[c][0]) * idx;
-      kx += 0.5 * k[c].hx *
-            (sq(-Du - q * s.ax[0] * s.v[c][0]) + sq(-Du - q * s.ax[1] * s.v[c][1]) +
-             sq(Dv - q * s.ax[0] * s.u[c][0]) + sq(Dv - q * s.ax[1] * s.u[c][1]));
-    }
-    if (bitof(sc, 2)) {
-      const double Du = (s.u[c][2] - s.u[c][0]) * idx, Dv = (s.v[c][2] - s.v[c][0]) * idx;
-      ky += 0.5 * k[c].hy *
-            (sq(-Du - q * s.ay[0] * s.v[c][0]) + sq(-Du - q * s.ay[3] * s.v[c][2]) +
-             sq(Dv - q * s.ay[0] * s.u[c][0]) + sq(Dv - q * s.ay[3] * s.u[c][2]));
-    }
+    e = fma(wx * k[c].hx, bond(s.u[c][0], s.v[c][0], s.ax[0], s.u[c][1], s.v[c][1], s.ax[1], q), e);
+    e = fma(wy * k[c].hy, bond(s.u[c][0], s.v[c][0], s.ay[0], s.u[c][2], s.v[c][2], s.ay[3], q), e);
   }
-  kx *= (bitof(sc, 1) * bitof(sc, 2) + bitof(sc, 6) * bitof(sc, 7)) * 0.5;
-  ky *= (bitof(sc, 0) * bitof(sc, 1) + bitof(sc, 3) * bitof(sc, 4)) * 0.5;
-  double em = 0;
   if (!nsf) {
     const double yf = (s.ay[1] - s.ay[0]) * idx, yb = (s.ay[0] - s.ay[2]) * idx;
     const double xf = (s.ax[3] - s.ax[0]) * idx, xb = (s.ax[0] - s.ax[4]) * idx;
-    if (bitof(cm, 0) && bitof(cm, 1) && bitof(cm, 2)) em += 0.125 * sq(yf - xf - s.h0);
-    if (bitof(cm, 2) && bitof(cm, 3) && bitof(cm, 4)) em += 0.125 * sq(yb - xf - s.h0);
-    if (bitof(cm, 4) && bitof(cm, 5) && bitof(cm, 6)) em += 0.125 * sq(yb - xb - s.h0);
-    if (bitof(cm, 6) && bitof(cm, 7) && bitof(cm, 0)) em += 0.125 * sq(yf - xb - s.h0);
+    const unsigned cq = quad_bits(cm);
+    const double e0 = yf - xf - s.h0, e1 = yb - xf - s.h0;
+    const double e2 = yb - xb - s.h0, e3 = yf - xb - s.h0;
+    double em = (cq & 0x01u) ? e0 * e0 : 0.0;
+    em = fma((cq & 0x04u) ? e1 : 0.0, e1, em);
+    em = fma((cq & 0x10u) ? e2 : 0.0, e2, em);
+    em = fma((cq & 0x40u) ? e3 : 0.0, e3, em);
+    e = fma(0.125, em, e);
   }
-  return ((kx + ky) + nl + em) * dx2;
+  return e * dx2;
 }
 
 // Magnetic field and supercurrents of one site, computeJBKernel
