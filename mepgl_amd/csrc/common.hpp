@@ -83,7 +83,7 @@ struct DevString {
   double* part_g;           // [F][ntiles][kPartG] workgroup partials
   double* part_p;           // [F][ntiles][kPartP]
   double* part_a;           // [F][ntiles][kPartA] arclength partials
-  double* cubic;            // [F][4] Thomas factors c', m, sub-diagonal, h
+  double* cubic;            // [F][kCubicCoefs] spline system
   void* cubic_rhs;          // cubic right-hand sides, the fields' layout in double
   int* plan_k;              // [F] linear redistribution: segment end node
   double* plan_w;           // [F] linear redistribution: weight of node k
@@ -103,6 +103,10 @@ struct WorkItem {
 // both domains and has no bond, quadrant or condensation term, so its
 // gradient, direction and line-search terms are exact zeros.
 constexpr int kItemNoBonds = 1;
+
+// Per image of a spline system: Thomas factors c' and m, sub-diagonal, spacing
+// h, 1 / m, 1 / h.
+constexpr int kCubicCoefs = 6;
 
 constexpr int kPartG = 4;   // g_norm2, g_delta_g (+ compensation terms)
 constexpr int kPartP = 10;  // A..E (+ compensation terms)

@@ -230,6 +230,7 @@ AuxArgs aux_args(mepgl_ctx* c) {
   a.out = c->d_out;
   a.jb = c->d_jb;
   a.only_string = -1;
+  for (auto& s : c->strings) a.most_images = std::max(a.most_images, s.dev.F);
   return a;
 }
 
@@ -637,8 +638,8 @@ int alloc_images(mepgl_ctx* c, StringHost& s, int F) {
   d.part_p = (double*)p;
   if ((rc = dev_alloc(c, &s, &p, nt * kPartA * sizeof(double)))) return rc;
   d.part_a = (double*)p;
-  if ((rc = dev_alloc(c, &s, &p, (size_t)F * 4 * sizeof(double)))) return rc;
-  HIP_TRY(c, hipMemsetAsync(p, 0, (size_t)F * 4 * sizeof(double), c->stream));
+  if ((rc = dev_alloc(c, &s, &p, (size_t)F * kCubicCoefs * sizeof(double)))) return rc;
+  HIP_TRY(c, hipMemsetAsync(p, 0, (size_t)F * kCubicCoefs * sizeof(double), c->stream));
   d.cubic = (double*)p;
   if ((rc = dev_alloc(c, &s, &p, (size_t)F * (2 * sizeof(int) + 2 * sizeof(double))))) return rc;
   HIP_TRY(c, hipMemsetAsync(p, 0, (size_t)F * (2 * sizeof(int) + 2 * sizeof(double)), c->stream));
@@ -970,7 +971,7 @@ int take_snapshot(mepgl_ctx* c, Snapshot& sn) {
     // recompute them, and a later redistribution must use the caller's.
     const size_t F = (size_t)s.dev.F;
     if ((rc = save(s.dev.plan_w, F * (2 * sizeof(int) + 2 * sizeof(double)))) ||
-        (rc = save(s.dev.cubic, F * 4 * sizeof(double))))
+        (rc = save(s.dev.cubic, F * kCubicCoefs * sizeof(double))))
       return rc;
   }
   const size_t scb = sizeof(ImageScalars) * c->total_images;

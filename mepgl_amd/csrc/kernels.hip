@@ -554,14 +554,28 @@ static void launch_arclen(const AuxArgs& a, hipStream_t st) {
   launch_arclen_upd<T, false>(a, st);
 }
 
+// The first node k >= 1 of F with s[k] >= x, or F - 1: what the reference's
+// incremental search stops at.  s does not decrease, so s[k] < x holds up to
+// some node and no further (for NaN it holds nowhere, as from the first NaN of
+// a running sum on).
+__device__ __forceinline__ int first_node(const double* s, int F, double x) {
+  int lo = 1, hi = F - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (s[mid] < x)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  return lo;
+}
+
 // computeArcLength (interpolation.cu:126-140) for both metrics, then the
 // linear redistribution plan of every new image on s_jb: the segment search
 // of generateNewFramesLinear (interpolation.cu:200-219).  One workgroup per
 // string.  The square roots run one image per thread; the prefix sums run in
 // one thread in the reference's order (so s and s_jb are the reference's
-// sums bit for bit); the segment searches run one new image per thread: for
-// a non-decreasing s the reference's incremental search stops at the first
-// node k >= 1 with s[k] >= s_new, which is what each thread finds directly.
+// sums bit for bit); the segment searches run one new image per thread.
 __global__ __launch_bounds__(kArcBlock) void k_arc_finalize(AuxArgs a, int nstrings) {
   __shared__ double ls[kMaxImages], lsj[kMaxImages];
   const int si = blockIdx.x;
@@ -599,8 +613,7 @@ __global__ __launch_bounds__(kArcBlock) void k_arc_finalize(AuxArgs a, int nstri
   // Linear plan (F_new = F).
   for (int n = tid; n < F; n += kArcBlock) {
     const double s_new = (double)n / ((double)F - 1);
-    int k = 1;
-    while (k + 1 < F && lsj[k] < s_new) ++k;
+    const int k = first_node(lsj, F, s_new);
     const double seg_start = k == 1 ? 0.0 : lsj[k - 1];
     s.plan_k[n] = k;
     s.plan_w[n] = (s_new - seg_start) / (lsj[k] - lsj[k - 1]);
@@ -621,7 +634,7 @@ __global__ __launch_bounds__(kArcBlock) void k_arc_finalize(AuxArgs a, int nstri
 // string, launched only before a cubic redistribution; the recurrences run
 // in one thread in the reference's order.
 __global__ __launch_bounds__(kArcBlock) void k_cubic_plan(AuxArgs a, int nstrings) {
-  __shared__ double lsj[kMaxImages], cum[kMaxImages];
+  __shared__ double lsj[kMaxImages], cum[kMaxImages], hs[kMaxImages + 1];
   const int si = blockIdx.x;
   if (si >= nstrings) return;
   const DevString& s = a.strings[si];
@@ -629,43 +642,90 @@ __global__ __launch_bounds__(kArcBlock) void k_cubic_plan(AuxArgs a, int nstring
   const int F = s.F;
   const int tid = threadIdx.x;
   if (F < 4 || F > kMaxImages) return;
-  double* cb = s.cubic;  // [F][4]: c', m, sub-diagonal, h
+  double* cb = s.cubic;  // [F][kCubicCoefs]
   for (int n = tid; n < F; n += kArcBlock) lsj[n] = sc[n].s_jb;
   __syncthreads();
-  for (int n = tid; n < F; n += kArcBlock) cb[4 * n + 3] = n == 0 ? 0.0 : lsj[n] - lsj[n - 1];
+  for (int n = tid; n <= F; n += kArcBlock) hs[n] = n == 0 || n == F ? 0.0 : lsj[n] - lsj[n - 1];
+  __syncthreads();
   if (tid == 0) {
-    auto h = [&](int n) { return n == 0 ? 0.0 : lsj[n] - lsj[n - 1]; };
+    double run = 0;
     cum[0] = 0;
-    for (int n = 1; n < F; ++n) cum[n] = cum[n - 1] + h(n);
-    double cprev = 0;
+#pragma unroll 8
+    for (int n = 1; n < F; ++n) {
+      run = run + hs[n];
+      cum[n] = run;
+    }
+  } else if (tid == kWave) {
+    // The factors, beside the running sums (another wavefront's).
+    double cprev = 0, h0 = 0, h1 = hs[1];
     for (int n = 0; n < F; ++n) {
+      const double h2 = hs[min(n + 2, F)];
       double dl, d, du;
       if (n == 0) {
-        dl = 0; d = -h(1); du = h(1);
+        dl = 0; d = -h1; du = h1;
       } else if (n == F - 1) {
-        dl = h(F - 1); d = -h(F - 1); du = 0;
+        dl = h0; d = -h0; du = 0;
       } else {
-        dl = h(n); d = 2 * (h(n) + h(n + 1)); du = h(n + 1);
+        dl = h0; d = 2 * (h0 + h1); du = h1;
       }
       const double m = n == 0 ? d : d - dl * cprev;
       cprev = du / m;
-      cb[4 * n + 0] = cprev;
-      cb[4 * n + 1] = m;
-      cb[4 * n + 2] = dl;
+      double* const q = cb + kCubicCoefs * n;
+      q[0] = cprev;
+      q[1] = m;
+      q[2] = dl;
+      h0 = h1;
+      h1 = h2;
     }
   }
   __syncthreads();
   for (int n = tid; n < F; n += kArcBlock) {
+    double* const q = cb + kCubicCoefs * n;
+    q[3] = hs[n];
+    q[4] = 1.0 / q[1];
+    q[5] = 1.0 / hs[n];
     const double s_new = (double)n / ((double)F - 1);
-    int k = 1;
-    while (k + 1 < F && cum[k] < s_new) ++k;
+    const int k = first_node(cum, F, s_new);
     s.cplan_k[n] = k;
     s.cplan_w[n] = (s_new - cum[k - 1]) / (lsj[k] - lsj[k - 1]);
   }
 }
 
 // generateNewFramesLinear (interpolation.cu:190-227) over all planes of a
-// string: image n of the output is w x[k] + (1 - w) x[k-1].
+// string: image n of the output is w x[k] + (1 - w) x[k-1].  Bound by the
+// fields' bytes, given enough loads in flight: a wavefront reads kLinearRows
+// rows of every plane of both images before it stores any of them.  One row
+// and plane at a time, with each store ahead of the next loads, it lived on
+// the number of wavefronts alone (65 two-component images of 200^2: FP64 63 us
+// at 4 rows per item, 80 at 19; mixed 28 and 44; now 63 and 28 at 19).
+constexpr int kLinearRows = 4;
+
+template <class T, int P0, int NP>
+__device__ __forceinline__ void linear_rows(const T* Xk, const T* Xk1, T* O, double w,
+                                            long long ps, long long pitch, int rows) {
+  for (int j0 = 0; j0 < rows; j0 += kLinearRows) {
+    T a[kLinearRows][NP], b[kLinearRows][NP];
+#pragma unroll
+    for (int r = 0; r < kLinearRows; ++r) {
+      const long long o = (long long)min(j0 + r, rows - 1) * pitch;
+#pragma unroll
+      for (int p = P0; p < NP; ++p) {
+        a[r][p] = Xk[p * ps + o];
+        b[r][p] = Xk1[p * ps + o];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < kLinearRows; ++r) {
+      if (j0 + r < rows) {
+        const long long o = (long long)(j0 + r) * pitch;
+#pragma unroll
+        for (int p = P0; p < NP; ++p)
+          O[p * ps + o] = (T)fma(w, (double)a[r][p], (1 - w) * (double)b[r][p]);
+      }
+    }
+  }
+}
+
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_redistribute_linear(AuxArgs a) {
   const WorkItem it = load_item(a.items, xcd_item(blockIdx.x, a.nitems));
@@ -674,17 +734,22 @@ __global__ __launch_bounds__(kBlock) void k_redistribute_linear(AuxArgs a) {
   if (t.i >= s.N) return;
   const int k = s.plan_k[t.n];
   const double w = s.plan_w[t.n];
-  const T* Xk = (const T*)s.x[a.xin] + (long long)k * s.image_stride;
+  const long long first = (long long)t.j0 * s.pitch + t.i, ps = s.plane_stride, pitch = s.pitch;
+  const T* Xk = (const T*)s.x[a.xin] + (long long)k * s.image_stride + first;
   const T* Xk1 = Xk - s.image_stride;
-  T* O = (T*)s.x[a.xout] + (long long)t.n * s.image_stride;
+  T* O = (T*)s.x[a.xout] + (long long)t.n * s.image_stride + first;
+  const int rows = t.j1 - t.j0;
   // A fixed and shared by every image stays as it is, in both buffers.
-  const int p0 = s.a_shared ? 2 : 0;
-  for (int j = t.j0; j < t.j1; ++j) {
-    const long long off = (long long)j * s.pitch + t.i;
-    for (int p = p0; p < s.nplanes; ++p) {
-      const long long o = p * s.plane_stride + off;
-      O[o] = (T)fma(w, (double)Xk[o], (1 - w) * (double)Xk1[o]);
-    }
+  if (s.nplanes == 6) {
+    if (s.a_shared)
+      linear_rows<T, 2, 6>(Xk, Xk1, O, w, ps, pitch, rows);
+    else
+      linear_rows<T, 0, 6>(Xk, Xk1, O, w, ps, pitch, rows);
+  } else {
+    if (s.a_shared)
+      linear_rows<T, 2, 4>(Xk, Xk1, O, w, ps, pitch, rows);
+    else
+      linear_rows<T, 0, 4>(Xk, Xk1, O, w, ps, pitch, rows);
   }
 }
 
@@ -706,6 +771,14 @@ __global__ __launch_bounds__(kBlock) void k_copy_a(AuxArgs a) {
   }
 }
 
+// x / m from r = 1 / m: the quotient corrected by its remainder, which gives
+// the bits of the division (Markstein) in a third of its operations.  Where
+// the product is not finite (m is zero or not finite), so is the division.
+__device__ __forceinline__ double div_by(double x, double m, double r) {
+  const double q = x * r;
+  return fma(fma(-q, m, x), r, q);
+}
+
 // redistributeCubic (interpolation.cu:292-481) in double, one spline system
 // per (site, plane): divided differences and end third differences
 // (computeDeltaX/Y), the Thomas solve of the system along the image axis (in
@@ -715,8 +788,156 @@ __global__ __launch_bounds__(kBlock) void k_copy_a(AuxArgs a) {
 //
 // The systems run along the image axis, so the F work items of a tile share
 // its (row, plane) pairs: item n takes pairs n, n + F, ..., and a thread
-// solves about rows * planes / F systems.  Every system's arithmetic and its
-// order are those of a sequential solve.
+// solves about rows * planes / F systems.
+//
+// A lane's right-hand sides stay in LDS (with the system's coefficients and the
+// new images' weights beside them), so memory sees the fields read, the second
+// time mostly from L2, and written.  What bounds it is the chain of the sweeps
+// at the few wavefronts that this LDS leaves a CU.  64 images of 256^2: 125 us
+// in FP64 and 99 in mixed precision (plan included), with the right-hand sides
+// in memory 226 and 146; 65 two-component images of 200^2: 151 and 129 against
+// 494 and 363.  Strings of up to kCubicLdsImages images: more would
+// leave too few wavefronts on a CU, and go through memory (k_redistribute_cubic).
+constexpr int kCubicLdsImages = 96;
+
+// LDS of one wavefront for F images.
+constexpr size_t cubic_lds(int F) {
+  return (size_t)F * (kWave * sizeof(double) + (kCubicCoefs + 4) * sizeof(double) + sizeof(int));
+}
+
+// The weights of a new image's spline value on f(k), f(k-1), sigma(k) and
+// sigma(k-1).
+struct SplineWeights {
+  double f1, f0, s1, s0;
+};
+__device__ __forceinline__ SplineWeights spline_weights(double w, double h, int textbook) {
+  const double wm = textbook ? ((1 - w) * (1 - w) * (1 - w) - (1 - w))
+                             : ((w - 1) * (w - 1) * (w - 1) - (w - 1));
+  return {w, 1 - w, h * h * (w * w * w - w), h * h * wm};
+}
+
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_redistribute_cubic_lds(AuxArgs a, int textbook) {
+  extern __shared__ double cubic_mem[];
+  const WorkItem it = load_item(a.items, xcd_item(blockIdx.x, a.nitems));
+  const DevString& s = a.strings[it.string];
+  const Strip t = strip_of(s, it);
+  const int F = s.F, p0 = s.a_shared ? 2 : 0, NP = s.nplanes - p0;
+  const int pairs = (t.j1 - t.j0) * NP, lane = t.lane;
+  if (t.n >= pairs) return;  // the whole wavefront
+  double* const D = cubic_mem + lane;                        // [F][64]
+  double* const co = cubic_mem + F * kWave;                  // [F][kCubicCoefs]
+  SplineWeights* const wt = (SplineWeights*)(co + F * kCubicCoefs);  // [F]
+  int* const pk = (int*)(wt + F);                            // [F]
+  for (int q = lane; q < F * kCubicCoefs; q += kWave) co[q] = s.cubic[q];
+  for (int n = lane; n < F; n += kWave) {
+    const int k = s.cplan_k[n];
+    pk[n] = k;
+    wt[n] = spline_weights(s.cplan_w[n], s.cubic[kCubicCoefs * k + 3], textbook);
+  }
+  __syncthreads();
+  const long long IS = s.image_stride, PS = s.plane_stride, PT = s.pitch;
+  const T* X = (const T*)s.x[a.xin];
+  T* Y = (T*)s.x[a.xout];
+  const bool live = t.i < s.N;
+  auto h = [&](int n) { return co[kCubicCoefs * n + 3]; };
+  // Each pass runs in batches of B images without a branch inside, so that a
+  // batch's reads of LDS and memory are in flight together, then singly.
+  constexpr int B = 8;
+  auto batches = [&](int n, int end, auto body) {
+    for (; n + B <= end; n += B) body(n, std::integral_constant<int, B>());
+    for (; n < end; ++n) body(n, std::integral_constant<int, 1>());
+  };
+  for (int q = t.n; q < pairs; q += F) {
+    const int j = t.j0 + q / NP, p = p0 + q % NP;
+    const long long off = p * PS + (long long)j * PT + t.ic;
+    const T* Xp = X + off;
+    T* O = Y + off;
+    auto f = [&](int n) { return (double)Xp[(long long)n * IS]; };
+    auto dl = [&](int n, double f1, double f0) {
+      return div_by(f1 - f0, h(n), co[kCubicCoefs * n + 5]);
+    };
+    // The end conditions need the first and last three differences.
+    double d3s, d3e, dprev, fprev;
+    {
+      const double f0 = f(0), f1 = f(1), f2 = f(2), f3 = f(3);
+      const double e0 = f(F - 4), e1 = f(F - 3), e2 = f(F - 2), e3 = f(F - 1);
+      const double d1 = dl(1, f1, f0), d2 = dl(2, f2, f1), d3 = dl(3, f3, f2);
+      const double g3 = dl(F - 3, e1, e0), g2 = dl(F - 2, e2, e1), g1 = dl(F - 1, e3, e2);
+      d3s = ((d3 - d2) / (h(3) + h(2)) - (d2 - d1) / (h(2) + h(1))) / (h(3) + h(2) + h(1));
+      d3e = ((g1 - g2) / (h(F - 1) + h(F - 2)) - (g2 - g3) / (h(F - 2) + h(F - 3))) /
+            (h(F - 1) + h(F - 2) + h(F - 3));
+      dprev = d1;
+      fprev = f1;
+    }
+    // The right-hand side dl(n+1) - dl(n) and the Thomas forward sweep.
+    auto sweep = [&](int n, double rhs, double prev) {
+      const double* const k = co + kCubicCoefs * n;
+      return div_by(rhs - k[2] * prev, k[1], k[4]);
+    };
+    double prev = sweep(0, h(1) * h(1) * d3s, 0.0);
+    D[0] = prev;
+    batches(1, F - 1, [&](int n0, auto count) {
+      constexpr int C = decltype(count)::value;
+      double dn[C];
+#pragma unroll
+      for (int i = 0; i < C; ++i) dn[i] = f(n0 + i + 1);
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const double fnext = dn[i];
+        dn[i] = dl(n0 + i + 1, fnext, fprev);
+        fprev = fnext;
+      }
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        prev = sweep(n0 + i, dn[i] - dprev, prev);
+        D[(n0 + i) * kWave] = prev;
+        dprev = dn[i];
+      }
+    });
+    prev = sweep(F - 1, -(h(F - 1) * h(F - 1)) * d3e, prev);
+    D[(F - 1) * kWave] = prev;
+    // Back substitution, from image F - 2 down.
+    batches(0, F - 1, [&](int m0, auto count) {
+      constexpr int C = decltype(count)::value;
+      const int n0 = F - 2 - m0;
+      double v[C], c[C];
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        v[i] = D[(n0 - i) * kWave];
+        c[i] = co[kCubicCoefs * (n0 - i)];
+      }
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        prev = v[i] - c[i] * prev;
+        D[(n0 - i) * kWave] = prev;
+      }
+    });
+    // The new images.
+    batches(0, F, [&](int n0, auto count) {
+      constexpr int C = decltype(count)::value;
+      T f1[C], f0[C];
+      double s1[C], s0[C];
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const int k = __builtin_amdgcn_readfirstlane(pk[n0 + i]);
+        f1[i] = Xp[(long long)k * IS];
+        f0[i] = Xp[(long long)(k - 1) * IS];
+        s1[i] = D[k * kWave];
+        s0[i] = D[(k - 1) * kWave];
+      }
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const SplineWeights w = wt[n0 + i];
+        const double v = w.f1 * (double)f1[i] + w.f0 * (double)f0[i] + (w.s1 * s1[i] + w.s0 * s0[i]);
+        if (live) O[(long long)(n0 + i) * IS] = (T)v;
+      }
+    });
+  }
+}
+
+// The same with the right-hand sides in memory, in the fields' layout in
+// double, for strings of more images.
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_redistribute_cubic(AuxArgs a, int textbook) {
   const WorkItem it = load_item(a.items, xcd_item(blockIdx.x, a.nitems));
@@ -734,13 +955,14 @@ __global__ __launch_bounds__(kBlock) void k_redistribute_cubic(AuxArgs a, int te
   T* Y = (T*)s.x[a.xout];
   double* Dl = (double*)s.cubic_rhs;  // in the fields' layout, in double
   const int pairs = (t.j1 - t.j0) * NP;
+  constexpr int C = kCubicCoefs;
   for (int q = t.n; q < pairs; q += F) {
     const int j = t.j0 + q / NP, p = p0 + q % NP;
     const long long off = p * PS + (long long)j * PT + t.i;
     const T* Xp = X + off;
     auto f = [&](int n) { return (double)Xp[(long long)n * IS]; };
     auto D = [&](int n) -> double& { return Dl[(long long)n * IS + off]; };
-    auto h = [&](int n) { return cb[4 * n + 3]; };
+    auto h = [&](int n) { return cb[C * n + 3]; };
     // First differences dl(n) = (f(n) - f(n-1)) / h(n); the end conditions
     // need only the first and last three.
     auto dl = [&](int n) { return (f(n) - f(n - 1)) / h(n); };
@@ -759,29 +981,26 @@ __global__ __launch_bounds__(kBlock) void k_redistribute_cubic(AuxArgs a, int te
     for (int n = 1; n < F - 1; ++n) {
       const double dnext = dl(n + 1);
       const double rhs = dnext - dprev;
-      prev = (rhs - cb[4 * n + 2] * prev) / cb[4 * n + 1];
+      prev = (rhs - cb[C * n + 2] * prev) / cb[C * n + 1];
       D(n) = prev;
       dprev = dnext;
     }
     {
       const double rhs = -(h(F - 1) * h(F - 1)) * d3e;
-      prev = (rhs - cb[4 * (F - 1) + 2] * prev) / cb[4 * (F - 1) + 1];
+      prev = (rhs - cb[C * (F - 1) + 2] * prev) / cb[C * (F - 1) + 1];
       D(F - 1) = prev;
     }
     double next = prev;
     for (int n = F - 2; n >= 0; --n) {
-      next = D(n) - cb[4 * n + 0] * next;
+      next = D(n) - cb[C * n + 0] * next;
       D(n) = next;
     }
     T* O = Y + off;
     for (int n = 0; n < F; ++n) {
       const int k = ck[n];
-      const double w = cw[n];
-      const double wm = textbook ? ((1 - w) * (1 - w) * (1 - w) - (1 - w))
-                                 : ((w - 1) * (w - 1) * (w - 1) - (w - 1));
-      const double v = w * f(k) + (1 - w) * f(k - 1) +
-                       h(k) * h(k) * ((w * w * w - w) * D(k) + wm * D(k - 1));
-      O[(long long)n * IS] = (T)v;
+      const SplineWeights w = spline_weights(cw[n], h(k), textbook);
+      O[(long long)n * IS] =
+          (T)(w.f1 * f(k) + w.f0 * f(k - 1) + (w.s1 * D(k) + w.s0 * D(k - 1)));
     }
   }
 }
@@ -797,19 +1016,32 @@ __device__ void align_body(const AuxArgs& a, const DevString& s, const WorkItem&
   if (t.n > 0 && t.i < s.N) {
     const T* X1 = (const T*)s.x[a.xin] + (long long)t.n * s.image_stride;
     const T* X0 = X1 - s.image_stride;
-    for (int j = t.j0; j < t.j1; ++j) {
-      const long long off = (long long)j * s.pitch + t.i;
-      double re = 0, im = 0;
+    const long long ps = s.plane_stride, pitch = s.pitch;
+    constexpr int R = 4;  // rows read ahead of their sums
+    for (int j = t.j0; j < t.j1; j += R) {
+      T u1[R][NC], v1[R][NC], u0[R][NC], v0[R][NC];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const long long pu = (PU1 + 2 * c) * s.plane_stride + off;
-        const long long pv = (PV1 + 2 * c) * s.plane_stride + off;
-        const double u1 = X1[pu], v1 = X1[pv], u0 = X0[pu], v0 = X0[pv];
-        re += u1 * u0 + v1 * v0;
-        im += u1 * v0 - v1 * u0;
+      for (int r = 0; r < R; ++r) {
+        const long long off = (long long)min(j + r, t.j1 - 1) * pitch + t.i;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const long long pu = (PU1 + 2 * c) * ps + off, pv = (PV1 + 2 * c) * ps + off;
+          u1[r][c] = X1[pu], v1[r][c] = X1[pv], u0[r][c] = X0[pu], v0[r][c] = X0[pv];
+        }
       }
-      two_sum_acc(acc_s[0], acc_c[0], re);
-      two_sum_acc(acc_s[1], acc_c[1], im);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if (j + r >= t.j1) break;
+        double re = 0, im = 0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const double a1 = u1[r][c], b1 = v1[r][c], a0 = u0[r][c], b0 = v0[r][c];
+          re += a1 * a0 + b1 * b0;
+          im += a1 * b0 - b1 * a0;
+        }
+        two_sum_acc(acc_s[0], acc_c[0], re);
+        two_sum_acc(acc_s[1], acc_c[1], im);
+      }
     }
   }
   publish_partial<2, true>(acc_s, acc_c, s.part_a, t.n, t.tile, s.tiles_x * s.tiles_y);
@@ -860,16 +1092,21 @@ __global__ __launch_bounds__(kBlock) void k_align_apply(AuxArgs a) {
   const double th = a.sc[s.img0 + t.n].theta;
   const T cs = (T)cos(th), sn = (T)sin(th);
   T* bufs[4] = {(T*)s.x[a.xin], (T*)s.d[a.dcur], (T*)s.g[0], (T*)s.g[1]};
-  for (int b = 0; b < 4; ++b) {
-    T* B = bufs[b] + (long long)t.n * s.image_stride;
-    for (int j = t.j0; j < t.j1; ++j) {
-      const long long off = (long long)j * s.pitch + t.i;
-      for (int c = 0; c < s.nc; ++c) {
-        const long long pu = (PU1 + 2 * c) * s.plane_stride + off;
-        const long long pv = (PV1 + 2 * c) * s.plane_stride + off;
-        const T u = B[pu], v = B[pv];
-        B[pu] = u * cs - v * sn;
-        B[pv] = u * sn + v * cs;
+  const long long first = (long long)t.n * s.image_stride + t.i, ps = s.plane_stride;
+  const int nc = s.nc, pitch = s.pitch;
+  // The four buffers are distinct: a site's values are all read before any is
+  // written.
+  for (int j = t.j0; j < t.j1; ++j) {
+    const long long off = first + (long long)j * pitch;
+    for (int c = 0; c < nc; ++c) {
+      const long long pu = (PU1 + 2 * c) * ps + off, pv = (PV1 + 2 * c) * ps + off;
+      T u[4], v[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) u[b] = bufs[b][pu], v[b] = bufs[b][pv];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        bufs[b][pu] = u[b] * cs - v[b] * sn;
+        bufs[b][pv] = u[b] * sn + v[b] * cs;
       }
     }
   }
@@ -1005,7 +1242,11 @@ static hipError_t launch_aux_impl(const AuxArgs& a, int which, int arg, hipStrea
       if (a.nitems > 0) hipLaunchKernelGGL(k_redistribute_linear<T>, g, b, 0, st, a);
       break;
     case kKernelCubic:
-      if (a.nitems > 0) hipLaunchKernelGGL(k_redistribute_cubic<T>, g, b, 0, st, a, arg);
+      if (a.nitems <= 0) break;
+      if (a.most_images <= kCubicLdsImages)
+        hipLaunchKernelGGL(k_redistribute_cubic_lds<T>, g, b, cubic_lds(a.most_images), st, a, arg);
+      else
+        hipLaunchKernelGGL(k_redistribute_cubic<T>, g, b, 0, st, a, arg);
       break;
     case kKernelCopyA:
       if (a.nitems > 0) hipLaunchKernelGGL(k_copy_a<T>, g, b, 0, st, a);

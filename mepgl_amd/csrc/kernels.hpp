@@ -66,6 +66,7 @@ struct AuxArgs {
                         // gradient norms (beta = 0 on the next step)
   double* out;          // per global image (energy)
   double* const* jb;    // per string JB planes (device array of pointers)
+  int most_images;      // of any string
   int only_string;      // scalar maintenance: string index, or -1 for all
   int nc, pl;           // arclength, energy: class of every item in `items`
                         // (components, parameter planes)
