@@ -1094,22 +1094,29 @@ __global__ __launch_bounds__(kBlock) void k_align_apply(AuxArgs a) {
   T* bufs[4] = {(T*)s.x[a.xin], (T*)s.d[a.dcur], (T*)s.g[0], (T*)s.g[1]};
   const long long first = (long long)t.n * s.image_stride + t.i, ps = s.plane_stride;
   const int nc = s.nc, pitch = s.pitch;
-  // The four buffers are distinct: a site's values are all read before any is
-  // written.
-  for (int j = t.j0; j < t.j1; ++j) {
-    const long long off = first + (long long)j * pitch;
+  // A buffer at a time: the four together, 16 streams of a wavefront, took
+  // 7 us longer over 64 images of 256^2 in FP64, where the whole alignment takes 105.
+  constexpr int R = 4;  // rows read before they are written
+  for (int b = 0; b < 4; ++b)
     for (int c = 0; c < nc; ++c) {
-      const long long pu = (PU1 + 2 * c) * ps + off, pv = (PV1 + 2 * c) * ps + off;
-      T u[4], v[4];
+      T* const U = bufs[b] + first + (PU1 + 2 * c) * ps;
+      T* const V = bufs[b] + first + (PV1 + 2 * c) * ps;
+      for (int j = t.j0; j < t.j1; j += R) {
+        T u[R], v[R];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) u[b] = bufs[b][pu], v[b] = bufs[b][pv];
+        for (int r = 0; r < R; ++r) {
+          const long long off = (long long)min(j + r, t.j1 - 1) * pitch;
+          u[r] = U[off], v[r] = V[off];
+        }
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        bufs[b][pu] = u[b] * cs - v[b] * sn;
-        bufs[b][pv] = u[b] * sn + v[b] * cs;
+        for (int r = 0; r < R; ++r) {
+          if (j + r >= t.j1) break;
+          const long long off = (long long)(j + r) * pitch;
+          U[off] = u[r] * cs - v[r] * sn;
+          V[off] = u[r] * sn + v[r] * cs;
+        }
       }
     }
-  }
 }
 
 // Phase winding around the grid boundary of one image (gl_utils.py:10-41,
