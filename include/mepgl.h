@@ -249,7 +249,9 @@ int mepgl_set_scalars(mepgl_ctx *ctx, int string, int which, const double *value
  * another part's G (mostly memory traffic).  A context starts with 2 parts;
  * mepgl_autotune picks 2 or 4 together with the segment heights.  Splitting
  * applies when an outer iteration has more than one step, and not while
- * per-kernel timing is on.
+ * per-kernel timing is on; unless it is asked for, a context of few rows of 64
+ * sites (under 6,000 in FP64, 10,000 in mixed precision, over all images)
+ * keeps one sequence.
  * 0: one launch sequence.  1: split, with the current part count.  2 to 4:
  * split into that many parts.  Other values: MEPGL_ERR_ARG.
  * mepgl_get_control returns the part count, or 0 when not split.  Results are
@@ -307,12 +309,12 @@ int mepgl_synchronize(mepgl_ctx *ctx);
  * size (config.cuh:25-31, blockSizeX); here one wavefront marches a
  * 64-column strip down `rows` rows (heights of 3k + 1 rows waste no work).
  * mepgl_set_segment_rows sets one string's height (clamped to
- * [min(N, 4), N]).  mepgl_autotune times five rounds per candidate height
- * (4 .. 127) of an outer iteration of mode L with `steps` NLCG steps
- * (arclength, linear redistribution, the steps; only the steps when a string
- * has one image), each round visiting every candidate in turn, for each
- * class of strings with equal N, components and fixed-A setting.  It keeps
- * the height with the fastest round and restores the solver state, so
+ * [min(N, 4), N]; the library itself also picks 1 for small strings).
+ * mepgl_autotune times five rounds per candidate height (4 .. 127) of an
+ * outer iteration of mode L with `steps` NLCG steps (arclength, linear
+ * redistribution, the steps; only the steps when a string has one image),
+ * each round visiting every candidate in turn, for each class of strings
+ * with equal N, components and fixed-A setting.  It keeps the height with the fastest round and restores the solver state, so
  * tuning leaves fields, scalars and reparametrisation plans as it found
  * them; it needs device memory for one copy of the fields, gradients and
  * directions.  rows_out

@@ -74,6 +74,7 @@ struct mepgl_ctx {
   hipStream_t xs[kMaxParts] = {};
   hipEvent_t fork_ev = nullptr, join_evs[kMaxParts] = {};
   bool split_images = true;  // MEPGL_CONTROL_SPLIT_IMAGES
+  bool split_small = false;  // ... asked for: contexts of few row strips too
   int parts = 2;             // parts of a split sequence, 2..kMaxParts
   bool edge_exchange = true; // MEPGL_CONTROL_EDGE_EXCHANGE
   // Global ids of each part's images, for the finishing launches of a split
@@ -166,26 +167,69 @@ int min_rows(int N) { return std::min(N, 4); }
 int clamp_rows(int rows, int N) { return std::max(std::min(rows, N), min_rows(N)); }
 
 size_t max_tiles(const DevString& d) {
-  return (size_t)d.tiles_x * (size_t)((d.N + min_rows(d.N) - 1) / min_rows(d.N));
+  const int h = std::min(min_rows(d.N), d.seg_rows);
+  return (size_t)d.tiles_x * (size_t)((d.N + h - 1) / h);
 }
 
-// Segment heights the library picks from.  The G and P kernels march rows
+// Segment heights the autotuner picks from.  The G and P kernels march rows
 // in rotations of three after the first, so heights of 3k + 1 rows waste no
 // work (any other height pads its last rotation).
 constexpr int kRowChoices[] = {4, 7, 10, 13, 16, 19, 22, 25, 31, 64, 127};
 
-// Rows marched by one wavefront.  Taller segments re-read fewer halo rows;
-// shorter ones give more wavefronts per launch.  Pick the tallest segment
-// that still yields about eight wavefronts per SIMD (1024 SIMDs).
-int choose_rows(const mepgl_string_desc& d, long long total_images) {
-  if (d.segment_rows > 0) return clamp_rows(d.segment_rows, d.N);
-  const long long cols = (d.N + kTileX - 1) / kTileX;
-  for (int h : {64, 31, 16, 10, 7}) {
-    const long long items = cols * ((d.N + h - 1) / h) * total_images;
-    if (h <= d.N && items >= 8192) return h;
-  }
-  return std::min(d.N, 4);
+// Row strips of a string: rows of 64 columns over all its images.
+long long row_strips(const mepgl_string_desc& d) {
+  return ((long long)d.N + kTileX - 1) / kTileX * d.N * std::max(d.F, 0);
 }
+
+// Strings whose items one launch covers.
+std::tuple<int, bool, bool> item_class(const mepgl_string_desc& d) {
+  bool planes = false;
+  for (auto* p : {&d.a_1, &d.b_1, &d.m_xx_1, &d.m_yy_1, &d.a_2, &d.b_2, &d.m_xx_2, &d.m_yy_2, &d.h})
+    planes = planes || p->plane;
+  return {d.ncomp, d.no_self_field != 0, planes};
+}
+
+// Rows marched by one wavefront, when launches cover `strips` row strips.
+// Taller segments re-read fewer halo rows and pay a wavefront's start less
+// often; shorter ones give more wavefronts.  A launch lasts as long as its
+// most loaded SIMD (of 1024): with k wavefronts there, a row takes 0.4 + 0.5 k
+// of the time that it takes a wavefront alone, up to the wavefronts that fit
+// (4, or 3 with more registers), and a wavefront's start takes as long as 3
+// rows.  Over 42 strings of 40^2 to 512^2 sites, 8 to 64 images, one and two
+// components and both precisions, the height of the lowest such cost was on
+// average 1 % slower than the best of 1 to 31 rows, 9 % at most.  (The tallest
+// segment with 8192 wavefronts, or else 4 rows: 64 images of 256^2 in mixed
+// precision 115 us per step at 7 rows, 108 at 16; 15 images of 64^2 22 us at 4
+// rows, 15 at one.)  One row per wavefront only while an image has at most 64
+// tiles, so that the line search stays in G (fold_line_search).
+int choose_rows(const mepgl_string_desc& d, int precision, long long strips) {
+  if (d.segment_rows > 0) return clamp_rows(d.segment_rows, d.N);
+  const int fit = precision == MEPGL_MIXED && d.ncomp == 1 ? 4 : 3;
+  const double share = (double)strips / (double)std::max(row_strips(d), 1LL);
+  const long long cols = (d.N + kTileX - 1) / kTileX;
+  auto per_row = [](double k) { return std::max(1.0, 0.4 + 0.5 * k); };
+  int best = clamp_rows(4, d.N);
+  double least = INFINITY;
+  for (int h : {1, 4, 7, 10, 13, 16, 19, 22, 25, 31}) {
+    if (h > d.N || (h == 1 && cols * d.N > kWave)) continue;
+    const double k = share * (double)(cols * ((d.N + h - 1) / h) * d.F) / 1024;
+    const double full = std::floor(k / fit), rest = std::ceil(k - full * fit);
+    const double cost = (h + 3) * (full * per_row(fit) + (rest > 0 ? per_row(rest) : 0.0));
+    if (cost < least) {
+      least = cost;
+      best = h;
+    }
+  }
+  return best;
+}
+
+// Row strips from which the image parts run as sequences of their own: with
+// fewer, one sequence leaves SIMDs idle already, and each part's launches take
+// as long as the whole's (15 images of 64^2: 15 us per step in one sequence,
+// 19 in two; 32 of 96^2, 6144 strips: 31.5 us either way in FP64, 27.3 and 29.5
+// in mixed precision; 32 of 160^2, 15360 strips: 58 and 55 us in FP64 at 10
+// rows, 47 and 45 in mixed precision at 4).
+long long split_strips(int precision) { return precision == MEPGL_MIXED ? 10000 : 6000; }
 
 bool param_ok(const mepgl_param& p) { return p.plane != nullptr || std::isfinite(p.value); }
 
@@ -890,6 +934,13 @@ int gauge_align_all(mepgl_ctx* c) {
   return run_aux(c, a, kKernelAlignApply, 0);
 }
 
+bool splits(const mepgl_ctx* c) {
+  if (!c->split_images || c->split_small) return c->split_images;
+  long long strips = 0;
+  for (auto& s : c->strings) strips += row_strips(s.desc);
+  return strips >= split_strips(c->precision);
+}
+
 // One outer iteration of loop() (mepgl.cu:153-303).
 int outer_iteration(mepgl_ctx* c, int relax, char mode, int nlcg) {
   int rc;
@@ -904,7 +955,7 @@ int outer_iteration(mepgl_ctx* c, int relax, char mode, int nlcg) {
   const bool maxwell = mode == 'M';
   // The steps of the image parts run side by side (per-kernel timing
   // keeps one stream).
-  const bool split = c->split_images && relax > 1 && !c->timing.on;
+  const bool split = splits(c) && relax > 1 && !c->timing.on;
   if (split && (rc = fork_parts(c))) return rc;
   for (int k = 0; k < relax; ++k)
     if ((rc = nlcg_step(c, k, nlcg, maxwell ? 1 : 0, k + 1 < relax, split))) {
@@ -1106,8 +1157,9 @@ int mepgl_create(const mepgl_string_desc* strings, int n_strings, int precision,
       return MEPGL_ERR_HIP;
     }
 
-  long long total_img = 0;
-  for (int i = 0; i < n_strings; ++i) total_img += std::max(strings[i].F, 0);
+  // Row strips of each item class (build_items): a launch covers one class.
+  std::map<std::tuple<int, bool, bool>, long long> strips;
+  for (int i = 0; i < n_strings; ++i) strips[item_class(strings[i])] += row_strips(strings[i]);
 
   c->strings.resize(n_strings);
   for (int si = 0; si < n_strings; ++si) {
@@ -1134,7 +1186,7 @@ int mepgl_create(const mepgl_string_desc* strings, int n_strings, int precision,
     d.nsf = in.no_self_field ? 1 : 0;
     d.a_shared = d.nsf;  // the fields start at zero in every image
     d.poly_exact = (flags & MEPGL_POLY_EXACT) ? 1 : 0;
-    d.seg_rows = choose_rows(in, total_img);
+    d.seg_rows = choose_rows(in, precision, strips[item_class(in)]);
     d.tiles_x = (in.N + kTileX - 1) / kTileX;
     d.tiles_y = (in.N + d.seg_rows - 1) / d.seg_rows;
     s.ntiles = d.tiles_x * d.tiles_y;
@@ -1752,6 +1804,10 @@ int mepgl_set_control(mepgl_ctx* c, int key, int value) {
       break;
     case MEPGL_CONTROL_SPLIT_IMAGES:
       if (value < 0 || value > kMaxParts) return MEPGL_ERR_ARG;
+      if (c->split_small != (value != 0)) {
+        c->split_small = value != 0;
+        destroy_graphs(c);
+      }
       if (value >= 2 && value != c->parts) {
         HIP_TRY(c, hipSetDevice(c->device));
         c->parts = value;
@@ -1781,7 +1837,7 @@ int mepgl_get_control(mepgl_ctx* c, int key, int* value) {
     case MEPGL_CONTROL_RELAXATION_STEPS: *value = c->relax_steps.load(); break;
     case MEPGL_CONTROL_NLCG: *value = c->nlcg.load(); break;
     case MEPGL_CONTROL_FOLD_LINE_SEARCH: *value = c->fold_ls ? 1 : 0; break;
-    case MEPGL_CONTROL_SPLIT_IMAGES: *value = c->split_images ? c->parts : 0; break;
+    case MEPGL_CONTROL_SPLIT_IMAGES: *value = splits(c) ? c->parts : 0; break;
     case MEPGL_CONTROL_EDGE_EXCHANGE: *value = c->edge_exchange ? 1 : 0; break;
     default: return MEPGL_ERR_ARG;
   }
@@ -1869,10 +1925,10 @@ int mepgl_autotune(mepgl_ctx* c, int steps, int* rows_out) {
   c->timing.on = false;
   // The heights are tuned for each part count of a split sequence (2 and
   // kMaxParts), and the count whose tuned schedule runs fastest is kept with
-  // its heights.
+  // its heights.  A context that runs one sequence keeps it.
   const int parts0 = c->parts;
   std::vector<int> part_cand{c->parts};
-  if (c->split_images)
+  if (splits(c))
     for (int p : {2, kMaxParts})
       if (p != c->parts) part_cand.push_back(p);
   double best_score = INFINITY;
