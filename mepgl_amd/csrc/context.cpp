@@ -100,7 +100,7 @@ struct mepgl_ctx {
   };
   std::vector<Group> groups;
   double** d_jb = nullptr;
-  double* d_out = nullptr;
+  double* energies = nullptr;  // per global image, pinned host memory
   std::string err;
   int xp = 0, dp = 0;        // current field / direction buffers
   bool pending = false;      // an update x += alpha d is owed
@@ -271,7 +271,7 @@ AuxArgs aux_args(mepgl_ctx* c) {
   a.xin = c->xp;
   a.xout = 1 - c->xp;
   a.dcur = c->dp;
-  a.out = c->d_out;
+  a.out = c->energies;
   a.jb = c->d_jb;
   a.only_string = -1;
   for (auto& s : c->strings) a.most_images = std::max(a.most_images, s.dev.F);
@@ -393,7 +393,7 @@ FinishArgs finish_args(mepgl_ctx* c, int part = -1) {
   }
   f.sc = c->d_sc;
   f.ls = c->d_ls;
-  f.out = c->d_out;
+  f.out = c->energies;
   f.xin = c->xp;
   f.health = c->health;
   return f;
@@ -704,13 +704,13 @@ int alloc_scalars(mepgl_ctx* c) {
   c->total_images = img;
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   if (c->d_sc) (void)hipFree(c->d_sc);
-  if (c->d_out) (void)hipFree(c->d_out);
+  if (c->energies) (void)hipHostFree(c->energies);
   c->d_sc = nullptr;
-  c->d_out = nullptr;
+  c->energies = nullptr;
   HIP_TRY(c, hipMalloc(&c->d_sc, sizeof(ImageScalars) * img));
   HIP_TRY(c, hipMemsetAsync(c->d_sc, 0, sizeof(ImageScalars) * img, c->stream));
-  HIP_TRY(c, hipMalloc(&c->d_out, sizeof(double) * img));
-  HIP_TRY(c, hipMemsetAsync(c->d_out, 0, sizeof(double) * img, c->stream));
+  HIP_TRY(c, hipHostMalloc((void**)&c->energies, sizeof(double) * img, hipHostMallocDefault));
+  std::fill_n(c->energies, img, 0.0);
   std::vector<int2> map;
   for (size_t si = 0; si < c->strings.size(); ++si)
     for (int n = 0; n < c->strings[si].dev.F; ++n) map.push_back(make_int2((int)si, n));
@@ -1311,7 +1311,7 @@ void mepgl_destroy(mepgl_ctx* c) {
   (void)hipFree(c->d_ls);
   (void)hipFree(c->d_items);
   (void)hipFree(c->d_jb);
-  (void)hipFree(c->d_out);
+  if (c->energies) (void)hipHostFree(c->energies);
   for (auto e : c->timing.pool) (void)hipEventDestroy(e);
   for (auto e : c->iter_done)
     if (e) (void)hipEventDestroy(e);
@@ -1707,15 +1707,16 @@ int mepgl_loop(mepgl_ctx* c, int iterations, int relax, char mode, int nlcg) {
 int mepgl_get_scalars(mepgl_ctx* c, int si, int which, double* out) {
   if (!valid_string(c, si) || !out) return fail(c, MEPGL_ERR_ARG, "get_scalars: bad arguments");
   HIP_TRY(c, hipSetDevice(c->device));
-  if (int rc = settle_ls(c)) return rc;
   const DevString& d = c->strings[si].dev;
+  if (which == MEPGL_SCALAR_ENERGY) {  // written by the energy pass (k_finish_energy)
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    std::copy_n(c->energies + d.img0, d.F, out);
+    return MEPGL_OK;
+  }
+  if (int rc = settle_ls(c)) return rc;
   std::vector<ImageScalars> h(d.F);
   HIP_TRY(c, hipMemcpyAsync(h.data(), c->d_sc + d.img0, sizeof(ImageScalars) * d.F,
                             hipMemcpyDeviceToHost, c->stream));
-  std::vector<double> e(d.F);
-  if (which == MEPGL_SCALAR_ENERGY)
-    HIP_TRY(c, hipMemcpyAsync(e.data(), c->d_out + d.img0, sizeof(double) * d.F,
-                              hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   for (int n = 0; n < d.F; ++n) {
     const ImageScalars& x = h[n];
@@ -1732,7 +1733,6 @@ int mepgl_get_scalars(mepgl_ctx* c, int si, int which, double* out) {
       case MEPGL_SCALAR_THETA: out[n] = x.theta; break;
       case MEPGL_SCALAR_WINDING_1: out[n] = x.winding[0]; break;
       case MEPGL_SCALAR_WINDING_2: out[n] = x.winding[1]; break;
-      case MEPGL_SCALAR_ENERGY: out[n] = e[n]; break;
       case MEPGL_SCALAR_POLY:
         for (int q = 0; q < 4; ++q) out[4 * n + q] = x.poly[q];
         break;
