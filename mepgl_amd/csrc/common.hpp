@@ -75,6 +75,9 @@ struct DevString {
   // 0.5/m_xx, 0.5/m_yy (used when planes == 0).
   double kc[2][7];
   DevParam a[2], b[2], mxx[2], myy[2], h;
+  // With a parameter or applied-field plane: what the step kernels read of
+  // them, in the fields' storage type, row by row (k_derive_params).
+  void* prm;
   const uint16_t* nn;
   void* x[2];
   void* d[2];
@@ -103,6 +106,10 @@ struct WorkItem {
 // both domains and has no bond, quadrant or condensation term, so its
 // gradient, direction and line-search terms are exact zeros.
 constexpr int kItemNoBonds = 1;
+
+// Derived planes per component: 2a, b, 0.5/m_xx, 0.5/m_yy, a/b; the applied
+// field follows the last component's.
+constexpr int kParamPlanes = 5;
 
 // Per image of a spline system: Thomas factors c' and m, sub-diagonal, spacing
 // h, 1 / m, 1 / h.

@@ -1233,6 +1233,19 @@ int mepgl_create(const mepgl_string_desc* strings, int n_strings, int precision,
     UP(a_2, d.a[1]) UP(b_2, d.b[1]) UP(m_xx_2, d.mxx[1]) UP(m_yy_2, d.myy[1])
     UP(h, d.h)
 #undef UP
+    d.prm = nullptr;
+    if (d.planes || d.h.p) {
+      const size_t planes = (size_t)kParamPlanes * in.ncomp + 1;
+      if ((rc = dev_alloc(cp, &s, &d.prm, planes * in.N * d.plane_stride * (cp->fp32() ? 4 : 8)))) {
+        *out = c.release();
+        return rc;
+      }
+      const hipError_t pe = launch_derive_params(d, cp->fp32(), c->stream);
+      if (pe != hipSuccess) {
+        *out = c.release();
+        return fail(*out, MEPGL_ERR_HIP, std::string("parameter planes: ") + hipGetErrorString(pe));
+      }
+    }
     // Neighbour maps.
     void *dsc = nullptr, *dcm = nullptr, *nn = nullptr;
     const size_t db = (size_t)in.N * in.N * sizeof(int32_t);

@@ -1169,6 +1169,30 @@ __global__ __launch_bounds__(kBlock) void k_finish_align(FinishArgs f) {
 }
 
 // ---------------------------------------------------------------------------
+// The planes that the step kernels read of a string with parameter or applied
+// field planes: evaluated in double and rounded once, as load_comp_const does.
+// Evaluated per row and image by the kernels, their divisions and conversions
+// were a third of the step's time in mixed precision: 33 two-component images
+// of 256^2 took 137 us per step, and 106 with the planes derived once (FP64, where
+// memory hides more of it: 195 and 193; of 129^2 77 and 71.5, mixed 61 and 46).
+template <class T>
+__global__ __launch_bounds__(64) void k_derive_params(DevString s) {
+  const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y;
+  if (i >= s.N) return;
+  const long long o = (long long)j * s.pitch + i, plane = s.plane_stride;
+  T* const p = (T*)s.prm + j * (kParamPlanes * s.nc + 1) * plane + i;
+  for (int c = 0; c < s.nc; ++c) {
+    const double a = param_at<T>(s.a[c], o), b = param_at<T>(s.b[c], o);
+    T* const k = p + kParamPlanes * c * plane;
+    k[0] = (T)(2.0 * a);
+    k[plane] = (T)b;
+    k[2 * plane] = (T)(0.5 / param_at<T>(s.mxx[c], o));
+    k[3 * plane] = (T)(0.5 / param_at<T>(s.myy[c], o));
+    k[4 * plane] = (T)(a / b);
+  }
+  p[kParamPlanes * s.nc * plane] = (T)hval(s, o);
+}
+
 // buildNearestNeighbourMap (nlcg.cu:48-103) for the superconducting (low
 // byte) and computational (high byte) domains of one string.
 __global__ void k_nn_map(const int* sc_dom, const int* comp_dom, int N, int pitch,
@@ -1314,6 +1338,15 @@ hipError_t launch_finish(const FinishArgs& f, int which, bool fp32, hipStream_t 
     default:
       return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_derive_params(const DevString& s, bool fp32, hipStream_t st) {
+  const dim3 g((s.N + 63) / 64, s.N), b(64);
+  if (fp32)
+    hipLaunchKernelGGL(k_derive_params<float>, g, b, 0, st, s);
+  else
+    hipLaunchKernelGGL(k_derive_params<double>, g, b, 0, st, s);
   return hipGetLastError();
 }
 

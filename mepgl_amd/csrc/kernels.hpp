@@ -92,6 +92,8 @@ template <class T, int NC>
 hipError_t launch_step_nc(const StepArgs& a, int which, hipStream_t st);
 hipError_t launch_finish(const FinishArgs& f, int which, bool fp32, hipStream_t st);
 hipError_t launch_aux(const AuxArgs& a, int which, int arg, bool fp32, hipStream_t st);
+// Fills DevString::prm.
+hipError_t launch_derive_params(const DevString& s, bool fp32, hipStream_t st);
 hipError_t launch_nn_map(const int* sc_dom, const int* comp_dom, int N, int pitch, uint16_t* nn,
                          hipStream_t st);
 hipError_t launch_fill(void* p, long long n, bool fp32, double v, hipStream_t st);

@@ -398,53 +398,76 @@ __device__ __forceinline__ uint16_t bload_u16(Rsrc r, unsigned vo) {
   return __builtin_amdgcn_raw_buffer_load_b16(r, vo, 0, 0);
 }
 
-// Per-site parameters of one row when some parameter is a plane: a, b,
-// m_xx, m_yy per component and the applied field at the five stencil
-// points (centre, +x, -x, +y, -y).
+// A string's derived parameter planes (DevString::prm, k_derive_params) as the
+// step kernels read them.  The 11 planes of a two-component string may take up
+// to 3.7 GiB where an image takes 2: offsets are unsigned.
 template <class T, int NC, bool PL>
-struct RowParams {
-  __device__ __forceinline__ void load(const ParamView<NC>&, gptr<const double>, long long, int,
-                                       int, int, const Strip&) {}
-};
+struct ParamBufs {};
 template <class T, int NC>
-struct RowParams<T, NC, true> {
-  double prm[NC][4];
-  T h[5];
-  __device__ __forceinline__ void load(const ParamView<NC>& pv, gptr<const double> hp, long long off,
-                                       int j, int N, int P_, const Strip& t) {
+struct ParamBufs<T, NC, true> {
+  Rsrc r;
+  unsigned ps, pitch;  // bytes between planes and between rows
+  T q[NC];
+};
+template <class T, int NC, bool PL>
+__device__ __forceinline__ ParamBufs<T, NC, PL> param_bufs(const DevString& s) {
+  ParamBufs<T, NC, PL> b;
+  if constexpr (PL) {
+    b.ps = (unsigned)(s.plane_stride * (long long)sizeof(T));
+    b.pitch = b.ps * (kParamPlanes * NC + 1);
+    b.r = __builtin_amdgcn_make_buffer_rsrc(s.prm, (short)0, (int)(b.pitch * (unsigned)s.N), kRsrcWord3);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) b.q[c] = uniform_value((T)s.q[c]);
+  }
+  return b;
+}
+
+// Per-site parameters of one row when some parameter is a plane: four of the
+// derived planes per component and the applied field, at the site (POLY, the P
+// kernel) or at the five stencil points (centre, +x, -x, +y, -y).
+template <class T, int NC, bool PL, bool POLY>
+struct RowParams {
+  __device__ __forceinline__ void load(const ParamBufs<T, NC, PL>&, int, int, const Strip&) {}
+  __device__ __forceinline__ void pin_values() {}
+};
+template <class T, int NC, bool POLY>
+struct RowParams<T, NC, true, POLY> {
+  static constexpr int H = POLY ? 1 : 5;
+  T prm[NC][4], h[H];
+  __device__ __forceinline__ void load(const ParamBufs<T, NC, true>& b, int j, int N,
+                                       const Strip& t) {
+    const unsigned row = (unsigned)j * b.pitch, o = (unsigned)(t.ic * (int)sizeof(T));
+    constexpr unsigned first = POLY ? 1 : 0;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        prm[c][k] = bload<T>(b.r, o, row + (kParamPlanes * c + first + k) * b.ps);
+    const unsigned hp = kParamPlanes * NC * b.ps;
+    h[0] = bload<T>(b.r, o, row + hp);
+    if constexpr (!POLY) {
+      h[1] = bload<T>(b.r, (unsigned)(min(t.ic + 1, N - 1) * (int)sizeof(T)), row + hp);
+      h[2] = bload<T>(b.r, (unsigned)(max(t.ic - 1, 0) * (int)sizeof(T)), row + hp);
+      h[3] = bload<T>(b.r, o, (unsigned)clampr(j + 1, N) * b.pitch + hp);
+      h[4] = bload<T>(b.r, o, (unsigned)clampr(j - 1, N) * b.pitch + hp);
+    }
+  }
+  __device__ __forceinline__ void pin_values();
+  // The constants of the row: G reads 2a, b, 0.5/m; P reads b, 0.5/m, a/b.
+  __device__ __forceinline__ void constants(const ParamBufs<T, NC, true>& b, CompConst<T> (&k)[NC]) const {
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      prm[c][0] = param_at<T>(pv.a[c], off);
-      prm[c][1] = param_at<T>(pv.b[c], off);
-      prm[c][2] = param_at<T>(pv.mxx[c], off);
-      prm[c][3] = param_at<T>(pv.myy[c], off);
-    }
-    if (hp) {
-      const int ip = min(t.ic + 1, N - 1), im = max(t.ic - 1, 0);
-      h[0] = (T)hp[off];
-      h[1] = (T)hp[(long long)j * P_ + ip];
-      h[2] = (T)hp[(long long)j * P_ + im];
-      h[3] = (T)hp[(long long)clampr(j + 1, N) * P_ + t.ic];
-      h[4] = (T)hp[(long long)clampr(j - 1, N) * P_ + t.ic];
+      constexpr int B = POLY ? 0 : 1;
+      k[c].q = b.q[c];
+      k[c].two_a = POLY ? (T)0 : prm[c][0];
+      k[c].b = prm[c][B];
+      k[c].two_b = k[c].b + k[c].b;
+      k[c].hx = prm[c][B + 1];
+      k[c].hy = prm[c][B + 2];
+      k[c].ab = POLY ? prm[c][3] : (T)0;
     }
   }
 };
-
-template <class T, int NC>
-__device__ __forceinline__ void comp_from_params(const double (&prm)[NC][4], const double (&q)[NC],
-                                                 CompConst<T> (&k)[NC]) {
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const double a = prm[c][0], b = prm[c][1], mx = prm[c][2], my = prm[c][3];
-    k[c].q = (T)q[c];
-    k[c].two_a = (T)(2.0 * a);
-    k[c].two_b = (T)(2.0 * b);
-    k[c].b = (T)b;
-    k[c].ab = (T)(a / b);
-    k[c].hx = (T)(0.5 / mx);
-    k[c].hy = (T)(0.5 / my);
-  }
-}
 
 // Byte offsets of a strip row: own column and halo column.
 struct RowOff {
@@ -461,6 +484,15 @@ __device__ __forceinline__ RowOff row_off(int row, int P_, const Strip& t) {
 template <class T>
 __device__ __forceinline__ void pin(T& v) {
   asm volatile("" : "+v"(v));
+}
+template <class T, int NC, bool POLY>
+__device__ __forceinline__ void RowParams<T, NC, true, POLY>::pin_values() {
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) pin(prm[c][k]);
+#pragma unroll
+  for (int k = 0; k < H; ++k) pin(h[k]);
 }
 // A compiler barrier for memory operations: later stores are not moved above
 // it (pinned computations before it stay before the stores).

@@ -44,7 +44,7 @@ struct GSide {
   static constexpr int P = 2 + 2 * NC;
   T go[P];
   T gst[NC][2];
-  RowParams<T, NC, PL> rp;
+  RowParams<T, NC, PL, false> rp;
 };
 
 // The old gradient is read unconditionally (the diagnostic entry point that
@@ -52,8 +52,7 @@ struct GSide {
 // data-dependent branches.
 template <class T, int NC, bool NSF, bool PL, bool MW>
 __device__ __forceinline__ void g_side_load(GSide<T, NC, PL>& sd, const GBufs& b, int row, int P_,
-                                            const Strip& t, const ParamView<NC>& pv,
-                                            gptr<const double> hp, int N) {
+                                            const Strip& t, const ParamBufs<T, NC, PL>& pb, int N) {
   const unsigned o = (unsigned)((row * P_ + t.ic) * (int)sizeof(T));
 #pragma unroll
   for (int p = 0; p < GSide<T, NC, PL>::P; ++p)
@@ -63,7 +62,7 @@ __device__ __forceinline__ void g_side_load(GSide<T, NC, PL>& sd, const GBufs& b
     sd.gst[q][0] = MW ? bload<T>(b.g, o, (PU1 + 2 * q) * b.ps) : (T)0;
     sd.gst[q][1] = MW ? bload<T>(b.g, o, (PV1 + 2 * q) * b.ps) : (T)0;
   }
-  sd.rp.load(pv, hp, (long long)row * P_ + t.ic, row, N, P_, t);
+  sd.rp.load(pb, row, N, t);
 }
 
 template <class T, int NC, bool PL>
@@ -72,14 +71,7 @@ __device__ __forceinline__ void pin_side(GSide<T, NC, PL>& sd) {
   for (int p = 0; p < GSide<T, NC, PL>::P; ++p) pin(sd.go[p]);
 #pragma unroll
   for (int q = 0; q < NC; ++q) pin(sd.gst[q][0]), pin(sd.gst[q][1]);
-  if constexpr (PL) {
-#pragma unroll
-    for (int q = 0; q < NC; ++q)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) pin(sd.rp.prm[q][k]);
-#pragma unroll
-    for (int k = 0; k < 5; ++k) pin(sd.rp.h[k]);
-  }
+  sd.rp.pin_values();
 }
 
 // In mixed precision G and P run as workgroups of kStepWaves wavefronts on
@@ -295,8 +287,7 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
   const T eta = (T)s.eta, gam = (T)s.gamma, del = (T)s.delta;
   CompConst<T> kconst[NC];
   if (!PL) load_comp_const<T, NC>(s, 0, kconst);
-  const ParamView<NC> pv = param_view<NC>(s);
-  gptr<const double> __restrict__ hp = as_global(s.h.p);
+  const auto pb = param_bufs<T, NC, PL>(s);
   const T hv = (T)s.h.v;
   double acc_s[2] = {0, 0}, acc_c[2] = {0, 0};
   constexpr int W = step_waves<T>();
@@ -412,7 +403,7 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
     process(w[1], raw, S1());
     g_batch<T, NC, UPD, NSF>(raw, b, clampr(jb + D, N), P_, t, hl);
     process(w[2], raw, S2());
-    g_side_load<T, NC, NSF, PL, MW>(sd[1], b, jb, P_, t, pv, hp, N);
+    g_side_load<T, NC, NSF, PL, MW>(sd[1], b, jb, P_, t, pb, N);
     // Row jb + D is finished at the first row's start.
     if (hp_.lds) edge_barrier();
     finish(w[0], S0());
@@ -435,7 +426,7 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
       const bool live = store && (UP ? j >= t.j0 : j < t.j1);
       if constexpr (BATCH) {
         g_batch<T, NC, UPD, NSF>(raw, b, clampr(j + 2 * D, N), P_, t, hl);
-        g_side_load<T, NC, NSF, PL, MW>(sd[IN], b, clampr(j + D, N), P_, t, pv, hp, N);
+        g_side_load<T, NC, NSF, PL, MW>(sd[IN], b, clampr(j + D, N), P_, t, pb, N);
       }
       // Row j + D, processed one row ago, takes its halo; row j's slot is as
       // full.
@@ -467,9 +458,9 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
       const GSide<T, NC, PL>& cur = sd[IC];
       CompConst<T> k[NC];
       if constexpr (PL) {
-        comp_from_params<T, NC>(cur.rp.prm, pv.q, k);
+        cur.rp.constants(pb, k);
 #pragma unroll
-        for (int q = 0; q < 5; ++q) nb.h[q] = hp ? cur.rp.h[q] : hv;
+        for (int q = 0; q < 5; ++q) nb.h[q] = cur.rp.h[q];
       } else {
 #pragma unroll
         for (int q = 0; q < NC; ++q) k[q] = kconst[q];
@@ -689,8 +680,7 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
 #pragma unroll
     for (int i = 0; i < (int)(sizeof(pconst) / sizeof(T)); ++i) v[i] = uniform_value(v[i]);
   }
-  const ParamView<NC> pv = param_view<NC>(s);
-  gptr<const double> __restrict__ hp = as_global(s.h.p);
+  const auto pb = param_bufs<T, NC, PL>(s);
   const T hv = (T)s.h.v * dx;
   double acc_s[5] = {0, 0, 0, 0, 0}, acc_c[5] = {0, 0, 0, 0, 0};
   // Everything the march needs from the string's descriptor is read above,
@@ -717,7 +707,7 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
     const int jb = UP ? t.j1 - 1 : t.j0;  // first row of the march
     PRaw<T, NC> raw;
     PRow<T, NC> w[3];
-    RowParams<T, NC, PL> rp[3];
+    RowParams<T, NC, PL, true> rp[3];
     // A row's raw loads into window values, d = -g + beta d
     // (computeStepDirection, nlcg.cu:985-993), and its slot of the ring.
     auto process = [&](PRow<T, NC>& w, const PRaw<T, NC>& r, auto slot_tag) {
@@ -769,7 +759,7 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
     process(w[1], raw, S1());
     p_load<T, NC, NSF>(raw, b, clampr(jb + D, N), P_, t, hl);
     process(w[2], raw, S2());
-    rp[1].load(pv, hp, (long long)jb * P_ + t.ic, jb, N, P_, t);
+    rp[1].load(pb, jb, N, t);
 
     // Row j: one batch of loads (the fields of row j + 2D, the parameters of
     // row j + D), the quartic of row j from registers, the batch into the
@@ -784,8 +774,7 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
       const bool live = store && (UP ? j >= t.j0 : j < t.j1);
       if constexpr (BATCH) {
         p_load<T, NC, NSF>(raw, b, clampr(j + 2 * D, N), P_, t, hl);
-        const int r1 = clampr(j + D, N);
-        rp[IN].load(pv, hp, (long long)r1 * P_ + t.ic, r1, N, P_, t);
+        rp[IN].load(pb, clampr(j + D, N), N, t);
       }
       // The neighbours' edges of row j, stored when they processed it, and
       // before row j + 2D's take the slot of row j - D.
@@ -832,9 +821,9 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
       nb.h0 = hv;
       if constexpr (PL) {
         CompConst<T> k[NC];
-        comp_from_params<T, NC>(rp[IC].prm, pv.q, k);
+        rp[IC].constants(pb, k);
         pc = poly_const<T, NC>(k, eta, gam, del, dx, dx2, exact);
-        if (hp) nb.h0 = rp[IC].h[0] * dx;
+        nb.h0 = rp[IC].h[0] * dx;
       }
 
       if (live) {
@@ -847,14 +836,7 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
       if constexpr (BATCH) {
         process(w[IP], raw, ip_tag);
         pin_row<T, NC>(w[IP]);
-        if constexpr (PL) {
-#pragma unroll
-          for (int q = 0; q < NC; ++q)
-#pragma unroll
-            for (int k2 = 0; k2 < 4; ++k2) pin(rp[IN].prm[q][k2]);
-#pragma unroll
-          for (int k2 = 0; k2 < 5; ++k2) pin(rp[IN].h[k2]);
-        }
+        rp[IN].pin_values();
         memory_fence_compiler();
       }
       __builtin_amdgcn_sched_barrier(0);
