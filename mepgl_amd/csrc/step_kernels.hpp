@@ -397,13 +397,21 @@ __device__ __forceinline__ void grad_body(const StepArgs& a, const DevString& s,
     GBatch<T, NC> raw;
     GWin<T, NC> w[3];
     GSide<T, NC, PL> sd[3];
-    g_batch<T, NC, UPD, NSF>(raw, b, clampr(jb - D, N), P_, t, hl);
-    process(w[0], raw, S0());
-    g_batch<T, NC, UPD, NSF>(raw, b, clampr(jb, N), P_, t, hl);
-    process(w[1], raw, S1());
-    g_batch<T, NC, UPD, NSF>(raw, b, clampr(jb + D, N), P_, t, hl);
-    process(w[2], raw, S2());
-    g_side_load<T, NC, NSF, PL, MW>(sd[1], b, jb, P_, t, pb, N);
+    // The first three rows are in flight together (one after another, 33
+    // two-component images of 129^2 took 41.9 us per step in mixed precision
+    // instead of 40.3, 15 images of 64^2 13.0 instead of 12.6; the march holds
+    // more registers than this).
+    {
+      GBatch<T, NC> r0, r1;
+      g_batch<T, NC, UPD, NSF>(r0, b, clampr(jb - D, N), P_, t, hl);
+      g_batch<T, NC, UPD, NSF>(r1, b, clampr(jb, N), P_, t, hl);
+      g_batch<T, NC, UPD, NSF>(raw, b, clampr(jb + D, N), P_, t, hl);
+      g_side_load<T, NC, NSF, PL, MW>(sd[1], b, jb, P_, t, pb, N);
+      __builtin_amdgcn_sched_barrier(0);
+      process(w[0], r0, S0());
+      process(w[1], r1, S1());
+      process(w[2], raw, S2());
+    }
     // Row jb + D is finished at the first row's start.
     if (hp_.lds) edge_barrier();
     finish(w[0], S0());
@@ -753,13 +761,17 @@ __device__ __forceinline__ void poly_body(const StepArgs& a, const DevString& s,
     auto edge = [&](auto slot_tag, int set, int p) {
       return ring[hp_.wave][decltype(slot_tag)::value][side][set][p];
     };
-    p_load<T, NC, NSF>(raw, b, clampr(jb - D, N), P_, t, hl);
-    process(w[0], raw, S0());
-    p_load<T, NC, NSF>(raw, b, clampr(jb, N), P_, t, hl);
-    process(w[1], raw, S1());
-    p_load<T, NC, NSF>(raw, b, clampr(jb + D, N), P_, t, hl);
-    process(w[2], raw, S2());
-    rp[1].load(pb, jb, N, t);
+    {  // the first three rows in flight together, as in the G loop
+      PRaw<T, NC> r0, r1;
+      p_load<T, NC, NSF>(r0, b, clampr(jb - D, N), P_, t, hl);
+      p_load<T, NC, NSF>(r1, b, clampr(jb, N), P_, t, hl);
+      p_load<T, NC, NSF>(raw, b, clampr(jb + D, N), P_, t, hl);
+      rp[1].load(pb, jb, N, t);
+      __builtin_amdgcn_sched_barrier(0);
+      process(w[0], r0, S0());
+      process(w[1], r1, S1());
+      process(w[2], raw, S2());
+    }
 
     // Row j: one batch of loads (the fields of row j + 2D, the parameters of
     // row j + D), the quartic of row j from registers, the batch into the
