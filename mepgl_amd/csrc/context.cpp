@@ -34,9 +34,14 @@ constexpr int kMaxParts = 4;
 
 namespace {
 
+// What a device allocation of a string is sized by: allocations per image are
+// made anew when the image count changes, the others stay.
+enum class Sized { kByString, kByImages };
+
 struct Alloc {
   void* p = nullptr;
   size_t bytes = 0;
+  Sized by = Sized::kByString;
 };
 
 struct StringHost {
@@ -138,7 +143,7 @@ int fail(mepgl_ctx* c, int code, const std::string& msg) {
       return fail(ctx, MEPGL_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-int dev_alloc(mepgl_ctx* c, StringHost* s, void** p, size_t bytes) {
+int dev_alloc(mepgl_ctx* c, StringHost* s, void** p, size_t bytes, Sized by) {
   *p = nullptr;
   if (bytes == 0) return MEPGL_OK;
   hipError_t e = hipMalloc(p, bytes);
@@ -147,17 +152,30 @@ int dev_alloc(mepgl_ctx* c, StringHost* s, void** p, size_t bytes) {
     return fail(c, MEPGL_ERR_NOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed: " +
                                         hipGetErrorString(e));
   }
-  if (s) s->owned.push_back({*p, bytes});
+  if (s) s->owned.push_back({*p, bytes, by});
   c->bytes += (long long)bytes;
   return MEPGL_OK;
 }
 
+void free_alloc(mepgl_ctx* c, const Alloc& a) {
+  (void)hipFree(a.p);
+  c->bytes -= (long long)a.bytes;
+}
+
 void free_string(mepgl_ctx* c, StringHost& s) {
-  for (auto& a : s.owned) {
-    (void)hipFree(a.p);
-    c->bytes -= (long long)a.bytes;
-  }
+  for (auto& a : s.owned) free_alloc(c, a);
   s.owned.clear();
+}
+
+void free_images(mepgl_ctx* c, StringHost& s) {
+  std::vector<Alloc> kept;
+  for (auto& a : s.owned) {
+    if (a.by == Sized::kByImages)
+      free_alloc(c, a);
+    else
+      kept.push_back(a);
+  }
+  s.owned.swap(kept);
 }
 
 // Shortest segment a schedule uses; the per-tile partial buffers are sized
@@ -647,7 +665,7 @@ int upload_param(mepgl_ctx* c, StringHost& s, const mepgl_param& p, DevParam& ou
   for (int j = 0; j < N; ++j)
     for (int i = 0; i < N; ++i) h[(size_t)j * P + i] = p.plane[(size_t)j * N + i];
   void* d;
-  int rc = dev_alloc(c, &s, &d, h.size() * sizeof(double));
+  int rc = dev_alloc(c, &s, &d, h.size() * sizeof(double), Sized::kByString);
   if (rc) return rc;
   HIP_TRY(c, hipMemcpyAsync(d, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice,
                             c->stream));
@@ -663,9 +681,9 @@ int alloc_images(mepgl_ctx* c, StringHost& s, int F) {
   const size_t fs = (size_t)F * d.image_stride * s.elem;
   for (int b = 0; b < 2; ++b) {
     int rc;
-    if ((rc = dev_alloc(c, &s, &d.x[b], fs))) return rc;
-    if ((rc = dev_alloc(c, &s, &d.d[b], fs))) return rc;
-    if ((rc = dev_alloc(c, &s, &d.g[b], fs))) return rc;
+    if ((rc = dev_alloc(c, &s, &d.x[b], fs, Sized::kByImages))) return rc;
+    if ((rc = dev_alloc(c, &s, &d.d[b], fs, Sized::kByImages))) return rc;
+    if ((rc = dev_alloc(c, &s, &d.g[b], fs, Sized::kByImages))) return rc;
     HIP_TRY(c, hipMemsetAsync(d.x[b], 0, fs, c->stream));
     HIP_TRY(c, hipMemsetAsync(d.d[b], 0, fs, c->stream));
     HIP_TRY(c, hipMemsetAsync(d.g[b], 0, fs, c->stream));
@@ -676,16 +694,18 @@ int alloc_images(mepgl_ctx* c, StringHost& s, int F) {
   const size_t nt = (size_t)F * max_tiles(d);
   void* p;
   int rc;
-  if ((rc = dev_alloc(c, &s, &p, nt * kPartG * sizeof(double)))) return rc;
+  if ((rc = dev_alloc(c, &s, &p, nt * kPartG * sizeof(double), Sized::kByImages))) return rc;
   d.part_g = (double*)p;
-  if ((rc = dev_alloc(c, &s, &p, nt * kPartP * sizeof(double)))) return rc;
+  if ((rc = dev_alloc(c, &s, &p, nt * kPartP * sizeof(double), Sized::kByImages))) return rc;
   d.part_p = (double*)p;
-  if ((rc = dev_alloc(c, &s, &p, nt * kPartA * sizeof(double)))) return rc;
+  if ((rc = dev_alloc(c, &s, &p, nt * kPartA * sizeof(double), Sized::kByImages))) return rc;
   d.part_a = (double*)p;
-  if ((rc = dev_alloc(c, &s, &p, (size_t)F * kCubicCoefs * sizeof(double)))) return rc;
+  if ((rc = dev_alloc(c, &s, &p, (size_t)F * kCubicCoefs * sizeof(double), Sized::kByImages))) return rc;
   HIP_TRY(c, hipMemsetAsync(p, 0, (size_t)F * kCubicCoefs * sizeof(double), c->stream));
   d.cubic = (double*)p;
-  if ((rc = dev_alloc(c, &s, &p, (size_t)F * (2 * sizeof(int) + 2 * sizeof(double))))) return rc;
+  if ((rc = dev_alloc(c, &s, &p, (size_t)F * (2 * sizeof(int) + 2 * sizeof(double)),
+                      Sized::kByImages)))
+    return rc;
   HIP_TRY(c, hipMemsetAsync(p, 0, (size_t)F * (2 * sizeof(int) + 2 * sizeof(double)), c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   d.plan_w = (double*)p;
@@ -824,7 +844,7 @@ int ensure_cubic_rhs(mepgl_ctx* c) {
   for (auto& s : c->strings) {
     if (s.dev.cubic_rhs) continue;
     int rc = dev_alloc(c, &s, &s.dev.cubic_rhs,
-                       (size_t)s.dev.F * s.dev.image_stride * sizeof(double));
+                       (size_t)s.dev.F * s.dev.image_stride * sizeof(double), Sized::kByImages);
     if (rc) return rc;
     changed = true;
   }
@@ -873,7 +893,7 @@ int ensure_dct(mepgl_ctx* c) {
       }
     for (int k = 0; k < N; ++k) h[(size_t)N * N + k] = 2.0 - 2.0 * std::cos(pi * k / N);
     void* p;
-    int rc = dev_alloc(c, &s, &p, h.size() * sizeof(double));
+    int rc = dev_alloc(c, &s, &p, h.size() * sizeof(double), Sized::kByString);
     if (rc) return rc;
     HIP_TRY(c, hipMemcpyAsync(p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice,
                               c->stream));
@@ -1236,7 +1256,8 @@ int mepgl_create(const mepgl_string_desc* strings, int n_strings, int precision,
     d.prm = nullptr;
     if (d.planes || d.h.p) {
       const size_t planes = (size_t)kParamPlanes * in.ncomp + 1;
-      if ((rc = dev_alloc(cp, &s, &d.prm, planes * in.N * d.plane_stride * (cp->fp32() ? 4 : 8)))) {
+      if ((rc = dev_alloc(cp, &s, &d.prm, planes * in.N * d.plane_stride * (cp->fp32() ? 4 : 8),
+                          Sized::kByString))) {
         *out = c.release();
         return rc;
       }
@@ -1249,8 +1270,9 @@ int mepgl_create(const mepgl_string_desc* strings, int n_strings, int precision,
     // Neighbour maps.
     void *dsc = nullptr, *dcm = nullptr, *nn = nullptr;
     const size_t db = (size_t)in.N * in.N * sizeof(int32_t);
-    if ((rc = dev_alloc(cp, &s, &nn, (size_t)in.N * d.pitch * sizeof(uint16_t))) ||
-        (rc = dev_alloc(cp, nullptr, &dsc, db)) || (rc = dev_alloc(cp, nullptr, &dcm, db))) {
+    if ((rc = dev_alloc(cp, &s, &nn, (size_t)in.N * d.pitch * sizeof(uint16_t), Sized::kByString)) ||
+        (rc = dev_alloc(cp, nullptr, &dsc, db, Sized::kByString)) ||
+        (rc = dev_alloc(cp, nullptr, &dcm, db, Sized::kByString))) {
       *out = c.release();
       return rc;
     }
@@ -1421,7 +1443,7 @@ int mepgl_gradient(mepgl_ctx* c, int si, double* a_g, double* p1_g, double* p2_g
   for (auto& s : c->strings) {
     if (s.dev.gs) continue;
     const size_t fs = (size_t)s.dev.F * s.dev.image_stride * s.elem;
-    if ((rc = dev_alloc(c, &s, &s.dev.gs, fs))) return rc;
+    if ((rc = dev_alloc(c, &s, &s.dev.gs, fs, Sized::kByImages))) return rc;
     HIP_TRY(c, hipMemsetAsync(s.dev.gs, 0, fs, c->stream));
     changed = true;
   }
@@ -1454,7 +1476,8 @@ int mepgl_compute_jb(mepgl_ctx* c, int si, double* b, double* j1, double* j2) {
     if (s.jb) continue;
     void* p;
     // b and j in the fields' layout (planes 0, 1 + 2c, 2 + 2c), in double.
-    if ((rc = dev_alloc(c, &s, &p, (size_t)s.dev.F * s.dev.image_stride * sizeof(double))))
+    if ((rc = dev_alloc(c, &s, &p, (size_t)s.dev.F * s.dev.image_stride * sizeof(double),
+                        Sized::kByImages)))
       return rc;
     s.jb = (double*)p;
     changed = true;
@@ -1554,22 +1577,7 @@ int mepgl_resample(mepgl_ctx* c, int si, int F_new) {
       n2[n * img + e] = std::fma(w, f2[o1], (1 - w) * f2[o0]);
     }
   }
-  // Free per-image buffers of this string (keep nn and parameter planes).
-  std::vector<Alloc> keep;
-  for (auto& a : s.owned) {
-    const void* p = a.p;
-    bool shared = p == (const void*)s.dev.nn;
-    const DevParam* prm[] = {&s.dev.a[0], &s.dev.b[0], &s.dev.mxx[0], &s.dev.myy[0], &s.dev.a[1],
-                             &s.dev.b[1], &s.dev.mxx[1], &s.dev.myy[1], &s.dev.h};
-    for (auto* q : prm) shared = shared || p == (const void*)q->p;
-    if (shared) {
-      keep.push_back(a);
-    } else {
-      (void)hipFree(a.p);
-      c->bytes -= (long long)a.bytes;
-    }
-  }
-  s.owned = keep;
+  free_images(c, s);
   if ((rc = alloc_images(c, s, F_new))) return rc;
   s.desc.F = F_new;
   destroy_graphs(c);
