@@ -314,13 +314,15 @@ int mepgl_synchronize(mepgl_ctx *ctx);
  * outer iteration of mode L with `steps` NLCG steps (arclength, linear
  * redistribution, the steps; only the steps when a string has one image),
  * each round visiting every candidate in turn, for each class of strings
- * with equal N, components and fixed-A setting.  It keeps the height with the fastest round and restores the solver state, so
- * tuning leaves fields, scalars and reparametrisation plans as it found
- * them; it needs device memory for one copy of the fields, gradients and
- * directions.  rows_out
- * (n_strings entries) may be NULL.  Sums over cells are taken per strip, so
- * a height change can move results in the last bits (well inside 1e-12
- * relative). */
+ * with equal N, components, fixed-A setting and parameter or applied-field
+ * planes or none; the height that a class's first string has is a candidate
+ * too.  A string whose partial sums have no room for a height takes the least
+ * that they have room for.  It keeps the height with the fastest round and
+ * restores the solver state, so tuning leaves fields, scalars and
+ * reparametrisation plans as it found them; it needs device memory for one
+ * copy of the fields, gradients and directions.  rows_out (n_strings entries)
+ * may be NULL.  Sums over cells are taken per strip, so a height change can
+ * move results in the last bits (well inside 1e-12 relative). */
 int mepgl_set_segment_rows(mepgl_ctx *ctx, int string, int rows);
 int mepgl_autotune(mepgl_ctx *ctx, int steps, int *rows_out);
 

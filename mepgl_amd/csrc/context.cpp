@@ -49,6 +49,7 @@ struct StringHost {
   DevString dev;            // host copy of the device descriptor
   std::vector<Alloc> owned; // device allocations of this string
   int ntiles = 0;
+  int part_rows = 1;        // least segment height the partial buffers hold
   std::vector<uint16_t> nn_host;  // neighbour map, [row][column] at the row pitch
   double* jb = nullptr;     // JB planes (lazy)
   double* dct = nullptr;    // DCT-II matrix and Laplacian eigenvalues (lazy)
@@ -178,16 +179,16 @@ void free_images(mepgl_ctx* c, StringHost& s) {
   s.owned.swap(kept);
 }
 
-// Shortest segment a schedule uses; the per-tile partial buffers are sized
-// for it, so a schedule change never reallocates.
+// Shortest segment a schedule is changed to.
 int min_rows(int N) { return std::min(N, 4); }
 
 int clamp_rows(int rows, int N) { return std::max(std::min(rows, N), min_rows(N)); }
 
-size_t max_tiles(const DevString& d) {
-  const int h = std::min(min_rows(d.N), d.seg_rows);
-  return (size_t)d.tiles_x * (size_t)((d.N + h - 1) / h);
-}
+// The per-tile partial buffers are sized for the shortest segment of a schedule
+// change, or for the string's own where that is shorter (choose_rows), so a
+// schedule change never reallocates; apply_schedule keeps every height at
+// least there.
+int least_rows(const DevString& d) { return std::min(min_rows(d.N), d.seg_rows); }
 
 // Segment heights the autotuner picks from.  The G and P kernels march rows
 // in rotations of three after the first, so heights of 3k + 1 rows waste no
@@ -691,7 +692,8 @@ int alloc_images(mepgl_ctx* c, StringHost& s, int F) {
   d.gs = nullptr;
   d.cubic_rhs = nullptr;
   s.jb = nullptr;
-  const size_t nt = (size_t)F * max_tiles(d);
+  s.part_rows = least_rows(d);
+  const size_t nt = (size_t)F * d.tiles_x * ((d.N + s.part_rows - 1) / s.part_rows);
   void* p;
   int rc;
   if ((rc = dev_alloc(c, &s, &p, nt * kPartG * sizeof(double), Sized::kByImages))) return rc;
@@ -988,12 +990,14 @@ int outer_iteration(mepgl_ctx* c, int relax, char mode, int nlcg) {
 
 // ---------------------------------------------------------------------------
 // Autotuning of the schedule: the segment height of each class of strings
-// (same N, components and fixed-A setting), timed on the live problem.
+// (same N, components, fixed-A setting and planes or none), timed on the live
+// problem.
 
 // Makes the descriptors, work list and graphs follow the strings' heights.
 int apply_schedule(mepgl_ctx* c) {
   for (auto& s : c->strings) {
     DevString& d = s.dev;
+    d.seg_rows = std::max(d.seg_rows, s.part_rows);
     d.tiles_y = (d.N + d.seg_rows - 1) / d.seg_rows;
     s.ntiles = d.tiles_x * d.tiles_y;
   }
@@ -1920,11 +1924,12 @@ int mepgl_autotune(mepgl_ctx* c, int steps, int* rows_out) {
   int rc = flush(c);
   if (rc) return rc;
   // Classes of strings that share a kernel specialisation and a grid size,
-  // tuned one after another, largest total work first.
-  std::map<std::tuple<int, int, int>, std::vector<int>> cls;
+  // tuned one after another, largest total work first.  A candidate below
+  // what a string's partial buffers hold is raised to that (apply_schedule).
+  std::map<std::pair<int, std::tuple<int, bool, bool>>, std::vector<int>> cls;
   for (size_t si = 0; si < c->strings.size(); ++si) {
-    const DevString& d = c->strings[si].dev;
-    cls[std::make_tuple(d.N, d.nc, d.nsf)].push_back((int)si);
+    const mepgl_string_desc& d = c->strings[si].desc;
+    cls[{d.N, item_class(d)}].push_back((int)si);
   }
   std::vector<std::pair<double, std::vector<int>>> order;
   for (auto& kv : cls) {

@@ -79,3 +79,54 @@ def test_resample_keeps_what_is_not_per_image(host, precision, planes):
         assert host.faults() == []
         assert sv.info(0)["bytes"] >= counted
     assert host.bytes() == before
+
+
+def solver_with_rows(strings, rows, **kw):
+    """A Solver whose strings take their segment heights from a list."""
+    from mepgl_amd.solver import Solver
+
+    class Uneven(Solver):
+        def _fill_desc(self, d, s, _):
+            super()._fill_desc(d, s, rows[[t is s for t in strings].index(True)])
+
+    return Uneven(strings, **kw)
+
+
+def square(F, planes, N=64):
+    return small_string(N=N, F=F, seed=F, planes=planes)
+
+
+# Strings of equal N of which one starts with one row per item and the other's
+# partial sums have room for heights from four on.
+UNEVEN = {
+    "planes": ([square(15, False), square(40, True)], [0, 0]),
+    "planes first": ([square(8, True), square(60, False)], [0, 0]),
+    "asked for": ([square(6, False), square(6, False)], [0, 4]),
+    "asked for, first": ([square(6, False), square(6, False)], [7, 0]),
+}
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("strings,rows", UNEVEN.values(), ids=UNEVEN)
+def test_tuned_heights_fit_the_partial_sums(host, strings, rows, precision):
+    with solver_with_rows(strings, rows, precision=precision, use_graph=False) as sv:
+        assert sorted(sv.info(i)["tile_rows"] == 1 for i in (0, 1)) == [False, True]
+        tuned = sv.autotune(2)
+        assert tuned == [sv.info(i)["tile_rows"] for i in (0, 1)]
+        sv.loop(1, 3, "L")
+        sv.computeFreeEnergy()
+        assert host.faults() == []
+
+
+def test_tuned_heights_after_a_resample(host):
+    """One string's partial sums are made anew at four rows, beside one that
+    still has one row."""
+    from mepgl_amd.solver import Solver
+
+    with Solver([square(6, False), square(5, False)], use_graph=False) as sv:
+        assert [sv.info(i)["tile_rows"] for i in (0, 1)] == [1, 1]
+        sv.set_segment_rows(1, 1)  # raised to four
+        sv.resample(1, 8)
+        sv.autotune(2)
+        sv.nlcgSteps(2)
+        assert host.faults() == []
