@@ -518,27 +518,27 @@ __device__ __forceinline__ double site_energy(const PolyNbhd<double, NC>& s,
     const double t3 = fma(-q0, u0, Dv), t4 = fma(-qn, un, Dv);
     return fma(t4, t4, fma(t3, t3, fma(t2, t2, t1 * t1)));
   };
-  // An absent bond (bits 0 and 2) has weight 0.
+  // Nothing of an absent bond (bits 0 and 2) or plaquette enters the sum: what
+  // lies outside the sample need not be finite (a mass of zero, A).
   const unsigned sp = pair_bits(sc);
-  const double wx = bitof(sc, 0) ? wx_fwd(sp) * 0.25 : 0.0;
-  const double wy = bitof(sc, 2) ? wy_fwd(sp) * 0.25 : 0.0;
+  const bool has_x = bitof(sc, 0), has_y = bitof(sc, 2);
+  const double wx = wx_fwd(sp) * 0.25, wy = wy_fwd(sp) * 0.25;
   double e = nl;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const double q = k[c].q;
-    e = fma(wx * k[c].hx, bond(s.u[c][0], s.v[c][0], s.ax[0], s.u[c][1], s.v[c][1], s.ax[1], q), e);
-    e = fma(wy * k[c].hy, bond(s.u[c][0], s.v[c][0], s.ay[0], s.u[c][2], s.v[c][2], s.ay[3], q), e);
+    const double bx = bond(s.u[c][0], s.v[c][0], s.ax[0], s.u[c][1], s.v[c][1], s.ax[1], q);
+    e = has_x ? fma(wx * k[c].hx, bx, e) : e;
+    const double by = bond(s.u[c][0], s.v[c][0], s.ay[0], s.u[c][2], s.v[c][2], s.ay[3], q);
+    e = has_y ? fma(wy * k[c].hy, by, e) : e;
   }
   if (!nsf) {
     const double yf = (s.ay[1] - s.ay[0]) * idx, yb = (s.ay[0] - s.ay[2]) * idx;
     const double xf = (s.ax[3] - s.ax[0]) * idx, xb = (s.ax[0] - s.ax[4]) * idx;
     const unsigned cq = quad_bits(cm);
-    const double e0 = yf - xf - s.h0, e1 = yb - xf - s.h0;
-    const double e2 = yb - xb - s.h0, e3 = yf - xb - s.h0;
-    double em = (cq & 0x01u) ? e0 * e0 : 0.0;
-    em = fma((cq & 0x04u) ? e1 : 0.0, e1, em);
-    em = fma((cq & 0x10u) ? e2 : 0.0, e2, em);
-    em = fma((cq & 0x40u) ? e3 : 0.0, e3, em);
+    const double e0 = (cq & 0x01u) ? yf - xf - s.h0 : 0.0, e1 = (cq & 0x04u) ? yb - xf - s.h0 : 0.0;
+    const double e2 = (cq & 0x10u) ? yb - xb - s.h0 : 0.0, e3 = (cq & 0x40u) ? yf - xb - s.h0 : 0.0;
+    const double em = fma(e3, e3, fma(e2, e2, fma(e1, e1, e0 * e0)));
     e = fma(0.125, em, e);
   }
   return e * dx2;
