@@ -558,9 +558,9 @@ static void launch_arclen(const AuxArgs& a, hipStream_t st) {
 }
 
 // The first node k >= 1 of F with s[k] >= x, or F - 1: what the reference's
-// incremental search stops at.  s does not decrease, so s[k] < x holds up to
-// some node and no further (for NaN it holds nowhere, as from the first NaN of
-// a running sum on).
+// incremental search stops at.  s must not decrease, so that s[k] < x holds up
+// to some node and no further (for NaN it holds nowhere, as from the first NaN
+// of a running sum on).
 __device__ __forceinline__ int first_node(const double* s, int F, double x) {
   int lo = 1, hi = F - 1;
   while (lo < hi) {
@@ -648,8 +648,12 @@ __global__ __launch_bounds__(kArcBlock) void k_cubic_plan(AuxArgs a, int nstring
   double* cb = s.cubic;  // [F][kCubicCoefs]
   for (int n = tid; n < F; n += kArcBlock) lsj[n] = sc[n].s_jb;
   __syncthreads();
-  for (int n = tid; n <= F; n += kArcBlock) hs[n] = n == 0 || n == F ? 0.0 : lsj[n] - lsj[n - 1];
-  __syncthreads();
+  int falls = 0;
+  for (int n = tid; n <= F; n += kArcBlock) {
+    hs[n] = n == 0 || n == F ? 0.0 : lsj[n] - lsj[n - 1];
+    falls |= hs[n] < 0;
+  }
+  falls = __syncthreads_or(falls);
   if (tid == 0) {
     double run = 0;
     cum[0] = 0;
@@ -688,7 +692,11 @@ __global__ __launch_bounds__(kArcBlock) void k_cubic_plan(AuxArgs a, int nstring
     q[4] = 1.0 / q[1];
     q[5] = 1.0 / hs[n];
     const double s_new = (double)n / ((double)F - 1);
-    const int k = first_node(cum, F, s_new);
+    int k = 1;
+    if (falls)  // an arclength given from outside need not rise
+      while (k + 1 < F && cum[k] < s_new) ++k;
+    else
+      k = first_node(cum, F, s_new);
     s.cplan_k[n] = k;
     s.cplan_w[n] = (s_new - cum[k - 1]) / (lsj[k] - lsj[k - 1]);
   }
