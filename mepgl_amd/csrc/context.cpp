@@ -210,11 +210,14 @@ std::tuple<int, bool, bool> item_class(const mepgl_string_desc& d) {
 
 // Rows marched by one wavefront, when launches cover `strips` row strips.
 // Taller segments re-read fewer halo rows and pay a wavefront's start less
-// often; shorter ones give more wavefronts.  A launch lasts as long as its
-// most loaded SIMD (of 1024): with k wavefronts there, a row takes 0.4 + 0.5 k
-// of the time that it takes a wavefront alone, up to the wavefronts that fit
-// (4, or 3 with more registers), and a wavefront's start takes as long as 3
-// rows.  Over 42 strings of 40^2 to 512^2 sites, 8 to 64 images, one and two
+// often; shorter ones give more wavefronts.  The model: a launch lasts as long
+// as its most loaded SIMD (of 1024), which takes its wavefronts in rounds of
+// `fit`; with k of them in a round a row takes 0.4 + 0.5 k of the time that it
+// takes a wavefront alone, and a wavefront's start takes as long as 3 rows.
+// All four constants are fitted to timings of whole steps; `fit` is no kernel's
+// occupancy (by its registers a SIMD holds 4 wavefronts of mixed G and P with
+// one component and 3 with two, but of FP64 G and P 3 and 2 with one component,
+// 2 and 1 with two, 1 each with two and planes).  Over 42 strings of 40^2 to 512^2 sites, 8 to 64 images, one and two
 // components and both precisions, the height of the lowest such cost was on
 // average 1 % slower than the best of 1 to 31 rows, 9 % at most.  (The tallest
 // segment with 8192 wavefronts, or else 4 rows: 64 images of 256^2 in mixed

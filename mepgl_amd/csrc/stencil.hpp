@@ -477,7 +477,7 @@ __device__ __forceinline__ Quartic<T> site_poly(const PolyNbhd<T, NC>& s,
     poly_bond(s.u[c][0], s.v[c][0], s.u[c][1], s.v[c][1], s.du[c][0], s.dv[c][0], s.du[c][1],
               s.dv[c][1], q * s.ax[0], q * s.ax[1], bx0, bx1, k.c1 * s.dax[0], k.c1 * s.dax[1], fx,
               fx, r);
-        poly_bond(s.u[c][0], s.v[c][0], s.u[c][2], s.v[c][2], s.du[c][0], s.dv[c][0], s.du[c][2],
+    poly_bond(s.u[c][0], s.v[c][0], s.u[c][2], s.v[c][2], s.du[c][0], s.dv[c][0], s.du[c][2],
               s.dv[c][2], q * s.ay[0], q * s.ay[3], by0, by3, -by0, -by3, k.hy * cy,
               k.hy3 * cy, r);
   }
